@@ -538,8 +538,9 @@ __global__ void __launch_bounds__(1024) k_prefill_dispatch(const uint32_t *__res
         uint32_t xb[kIdsPer];
         int rkb[kIdsPer];
         if (r0 > 0) {  // (the first batch's table was cleared at the start)
+            __syncthreads();  // the previous batch's reads of the table are done
             for (int q = tid; q < SB * E; q += 1024) tab[q] = 0;
-            __syncthreads();  // (also: the previous batch's reads of the table and cur's update are done)
+            __syncthreads();
         }
 #pragma unroll
         for (int rr = 0; rr < kIdsPer; rr++) {

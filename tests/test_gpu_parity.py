@@ -872,6 +872,29 @@ def test_gpu_prefill_large_batches(ctx, pool, T, E, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,k", [
+    (3000, 128, 8),   # 24,000 assignments: three tables of eight rounds
+    (2100, 256, 8),   # five tables of four rounds
+])
+def test_gpu_prefill_many_placement_tables(ctx, pool, T, E, k):
+    # the dispatch fills its placement table several times: a table is
+    # cleared for its next use only after every wavefront has read it
+    w = synth.moe_weights(85, 256, E, 64, down_cols=256)
+    router, gate_up, down = lt.upload_moe(ctx, w)
+    X = synth.normal(synth.stream(86, T), (T, 256))
+    out = np.zeros((T, 256), np.float32)
+    for _ in range(3):
+        prev = out.copy()
+        ctx.moe_prefill(out, X, router, gate_up, down, k, 64, norm_topk=True)
+    assert np.array_equal(prev.view(np.uint32), out.view(np.uint32))
+    sel = np.arange(0, T, 11)
+    ref, _, _ = orc.moe_prefill(w, X[sel], k, norm_topk=True, pool=pool)
+    assert rel_l2(out[sel], ref) <= PREFILL_REL_L2
+    for t in (router, gate_up, down):
+        t.free()
+
+
+@pytest.mark.gpu
 def test_gpu_prefill_one_token_chunks(ctx, cfg3, pool):
     # experts that get one token of the batch stream their weights against
     # the token's int8 limbs instead of an f16 tile; LT_PREFILL_NO_TINY
