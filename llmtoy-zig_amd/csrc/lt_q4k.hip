@@ -131,70 +131,7 @@ __device__ __forceinline__ float q4k_chunk_dot_limbs(uint4 hdr, uint4 q, int cc,
     return ((d * sc0) * dl - (dmin * mn0) * x.xs[0]) + ((d * sc1) * dh - (dmin * mn1) * x.xs[1]);
 }
 
-// Stage x[0..n) into LDS with 16-byte loads (n % 4 == 0).
-__device__ __forceinline__ void stage_x(float *xs, const float *x, int n) {
-    for (int i = threadIdx.x * 4; i < n; i += blockDim.x * 4)
-        *reinterpret_cast<float4 *>(xs + i) = *reinterpret_cast<const float4 *>(x + i);
-    __syncthreads();
-}
-
 }  // namespace
-
-// ------------------------------------------------------------------------
-// Generic matvec y[r] = W[row0 + r] . x for r < nrows.
-// G lanes per row (power of two), CPL chunks per lane, R rows per lane group.
-// Block: 256 threads = 256/G groups.  Grid: ceil(nrows / (groups * R)).
-template <int G, int CPL, int R>
-__global__ void __launch_bounds__(256) k_matvec_q4k(const uint8_t *__restrict__ hdr,
-                                                    const uint8_t *__restrict__ qs,
-                                                    const float *__restrict__ x, float *__restrict__ y,
-                                                    int row0, int nrows, int nsb) {
-    extern __shared__ float xs[];
-    stage_x(xs, x, nsb * 256);
-    const int groups = 256 / G;
-    const int g = threadIdx.x / G, lane = threadIdx.x % G;
-    const int rbase = (blockIdx.x * groups + g) * R;
-    const int nch = nsb * 8;
-    float acc[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) acc[r] = 0.f;
-#pragma unroll
-    for (int i = 0; i < CPL; i++) {
-        const int c = lane + G * i;
-        if (c < nch) {
-            const int sb = c >> 3, cc = c & 7;
-            uint4 hv[R], qv[R];
-#pragma unroll
-            for (int r = 0; r < R; r++) {
-                int row = rbase + r;
-                if (row < nrows) {
-                    size_t blk = (size_t)(row0 + row) * nsb + sb;
-                    hv[r] = ldg16(hdr + blk * 16);
-                    qv[r] = ldg16(qs + blk * 128 + cc * 16);
-                }
-            }
-            XChunk xc;
-            load_xchunk(xs, sb, cc, xc);
-            sum_xchunk(xc);
-#pragma unroll
-            for (int r = 0; r < R; r++)
-                if (rbase + r < nrows) acc[r] += q4k_chunk_dot(hv[r], qv[r], cc, xc);
-        }
-    }
-    if constexpr (G == 64) {
-        // row r's total lands in lanes [r*64/R, (r+1)*64/R)
-        const float t = wave_sum_transposed<R>(acc, lane, p32_first(lane));
-        constexpr int SH = R == 8 ? 3 : (R == 4 ? 4 : (R == 2 ? 5 : 6));
-        const int r = lane >> SH;
-        if ((lane & ((1 << SH) - 1)) == 0 && rbase + r < nrows) y[rbase + r] = t;
-    } else {
-#pragma unroll
-        for (int r = 0; r < R; r++) {
-            float v = group_sum<G>(acc[r]);
-            if (lane == 0 && rbase + r < nrows) y[rbase + r] = v;
-        }
-    }
-}
 
 // ------------------------------------------------------------------------
 // Streaming matvec for rows of NSB = 1, 2, 4, 8 or 16 super-blocks (config 2
@@ -227,7 +164,7 @@ constexpr int kQ4StreamND = 4;
 
 template <int NSB, int ND>
 __global__ void __launch_bounds__(256, q4k_stream_waves(ND)) k_matvec_q4k_stream(const uint8_t *hdr, const uint8_t *qs,
-                                                                                 const float *x, float *y, int row0,
+                                                                                 const float *x, float *y,
                                                                                  int nrows) {
     constexpr int PPR = 4 * NSB, LPR = PPR < 64 ? PPR : 64, UPL = PPR / LPR, RPS = 64 / LPR;
     __shared__ __attribute__((aligned(16))) uint32_t la[64 * NSB], lb[64 * NSB];
@@ -241,7 +178,7 @@ __global__ void __launch_bounds__(256, q4k_stream_waves(ND)) k_matvec_q4k_stream
     auto ld = [&](Q4Regs<UPL> &w, int rb) {
         int row = rb + rs;
         row = row < nrows ? row : nrows - 1;  // every load unconditional
-        const size_t b0 = (size_t)(row0 + row) * NSB;
+        const size_t b0 = (size_t)row * NSB;
 #pragma unroll
         for (int j = 0; j < UPL; j++) {
             const size_t blk = b0 + ((l + LPR * j) >> 2);
@@ -307,8 +244,8 @@ __global__ void __launch_bounds__(256, q4k_stream_waves(ND)) k_matvec_q4k_stream
 }
 
 template <int NSB>
-static hipError_t launch_q4k_stream(const DevTensor &W, size_t row0, size_t nrows, const float *x, float *y,
-                                    hipStream_t s) {
+static hipError_t launch_q4k_stream(const DevTensor &W, const float *x, float *y, hipStream_t s) {
+    const size_t nrows = W.total_rows;
     constexpr int LPR = 4 * NSB < 64 ? 4 * NSB : 64, RPS = 64 / LPR;
     const size_t slabs = (nrows + RPS - 1) / RPS;
     // Small matrices: four slabs per wave, all in flight from the start
@@ -319,56 +256,29 @@ static hipError_t launch_q4k_stream(const DevTensor &W, size_t row0, size_t nrow
     constexpr size_t nblk_big = (size_t)256 * q4k_stream_waves(kQ4StreamND);
     if (slabs >= nblk_big * 4 * 2 * kQ4StreamND) {
         hipLaunchKernelGGL((k_matvec_q4k_stream<NSB, kQ4StreamND>), dim3((unsigned)nblk_big), dim3(256), 0, s, W.p0,
-                           W.p1, x, y, (int)row0, (int)nrows);
+                           W.p1, x, y, (int)nrows);
     } else {
         constexpr size_t cap = (size_t)256 * q4k_stream_waves(4);
         size_t nblk = (slabs + 15) / 16;
         if (nblk > cap) nblk = cap;
         hipLaunchKernelGGL((k_matvec_q4k_stream<NSB, 4>), dim3((unsigned)nblk), dim3(256), 0, s, W.p0, W.p1, x, y,
-                           (int)row0, (int)nrows);
+                           (int)nrows);
     }
     return hipGetLastError();
 }
 
-template <int G, int CPL>
-static hipError_t launch_mv_q4k_t(const DevTensor &W, size_t row0, size_t nrows, const float *x, float *y,
-                                  hipStream_t s) {
-    constexpr int R = 4;
-    const int groups = 256 / G;
-    const int nblk = (int)((nrows + (size_t)groups * R - 1) / ((size_t)groups * R));
-    const int nsb = (int)W.blocks_per_row;
-    hipLaunchKernelGGL((k_matvec_q4k<G, CPL, R>), dim3(nblk), dim3(256), nsb * 256 * sizeof(float), s, W.p0, W.p1,
-                       x, y, (int)row0, (int)nrows, nsb);
-    return hipGetLastError();
-}
-
-hipError_t launch_matvec_q4k(const DevTensor &W, size_t row0, size_t nrows, const float *x, float *y,
-                             hipStream_t s) {
-    if ((row0 + nrows) * W.blocks_per_row < (size_t)1 << 31) {  // int row indices in the streaming kernel
+hipError_t launch_matvec_q4k(const DevTensor &W, const float *x, float *y, hipStream_t s) {
+    if (W.total_rows * W.blocks_per_row < (size_t)1 << 31) {  // int row indices in the streaming kernel
         switch (W.blocks_per_row) {
-        case 1: return launch_q4k_stream<1>(W, row0, nrows, x, y, s);
-        case 2: return launch_q4k_stream<2>(W, row0, nrows, x, y, s);
-        case 4: return launch_q4k_stream<4>(W, row0, nrows, x, y, s);
-        case 8: return launch_q4k_stream<8>(W, row0, nrows, x, y, s);
-        case 16: return launch_q4k_stream<16>(W, row0, nrows, x, y, s);
+        case 1: return launch_q4k_stream<1>(W, x, y, s);
+        case 2: return launch_q4k_stream<2>(W, x, y, s);
+        case 4: return launch_q4k_stream<4>(W, x, y, s);
+        case 8: return launch_q4k_stream<8>(W, x, y, s);
+        case 16: return launch_q4k_stream<16>(W, x, y, s);
         default: break;
         }
     }
-    const int nch = (int)W.blocks_per_row * 8;
-    if (nch <= 8) return launch_mv_q4k_t<8, 1>(W, row0, nrows, x, y, s);
-    if (nch <= 16) return launch_mv_q4k_t<16, 1>(W, row0, nrows, x, y, s);
-    if (nch <= 32) return launch_mv_q4k_t<32, 1>(W, row0, nrows, x, y, s);
-    switch ((nch + 63) / 64) {
-    case 1: return launch_mv_q4k_t<64, 1>(W, row0, nrows, x, y, s);
-    case 2: return launch_mv_q4k_t<64, 2>(W, row0, nrows, x, y, s);
-    case 3: return launch_mv_q4k_t<64, 3>(W, row0, nrows, x, y, s);
-    case 4: return launch_mv_q4k_t<64, 4>(W, row0, nrows, x, y, s);
-    case 5: return launch_mv_q4k_t<64, 5>(W, row0, nrows, x, y, s);
-    case 6: return launch_mv_q4k_t<64, 6>(W, row0, nrows, x, y, s);
-    case 7: return launch_mv_q4k_t<64, 7>(W, row0, nrows, x, y, s);
-    case 8: return launch_mv_q4k_t<64, 8>(W, row0, nrows, x, y, s);
-    default: return hipErrorInvalidValue;  // K > 16384: rejected by the API layer
-    }
+    return launch_matvec_rows(W, x, y, s);
 }
 
 // ------------------------------------------------------------------------

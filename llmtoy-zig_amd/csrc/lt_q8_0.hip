@@ -148,10 +148,6 @@ static hipError_t launch_q8_any(const DevTensor &A, const DevTensor *B, const fl
     }
 }
 
-hipError_t launch_matvec_q8_0(const DevTensor &W, const float *x, float *y, hipStream_t s) {
-    return launch_q8_any<false>(W, nullptr, x, y, 0, s);
-}
-
 hipError_t launch_gate_up_q8_0(const DevTensor &Wg, const DevTensor &Wu, const float *x, uint32_t act, float *h,
                                hipStream_t s) {
     return launch_q8_any<true>(Wg, &Wu, x, h, act, s);

@@ -284,6 +284,53 @@ def test_gpu_matvec_limb_nan(ctx, gtype, cols):
     assert np.isnan(y).all()
 
 
+@pytest.mark.parametrize("gtype,rows,cols", [
+    (ggml.Q8_0, 1, 32), (ggml.Q8_0, 131, 64),        # rows of one and two units, inside a wavefront
+    (ggml.Q8_0, 70, 2080), (ggml.Q8_0, 7001, 2816),  # 65 and 88 units: rows straddle wavefronts
+    (ggml.Q8_0, 40, 16384), (ggml.Q8_0, 1100, 16384),  # 512 units: one row a pass, one and three passes
+    (ggml.Q8_0, 16400, 512),                         # several rounds a workgroup, ragged last pass
+    (ggml.Q8_0, 30000, 96),
+    (ggml.Q4_K, 3, 768), (ggml.Q4_K, 1001, 2816), (ggml.Q4_K, 37, 16384), (ggml.Q4_K, 30000, 768),
+    (ggml.Q4_K, 300, 8192),                          # 32 super-blocks: 128 units
+    (ggml.Q6_K, 1, 768), (ggml.Q6_K, 999, 2816), (ggml.Q6_K, 37, 16384), (ggml.Q6_K, 30000, 768)])
+def test_gpu_matvec_any_row_length(ctx, pool, gtype, rows, cols):
+    # fp32 throughout: both sides round each of cols products and adds to
+    # 2^-24 in chains of at most cols / 32 terms (the oracle's), so their
+    # relative error is below 2^-24 sqrt(cols / 32) ~ 1.4e-6 each
+    g = np.random.default_rng(rows + cols)
+    w = synth.quant_matrix(g, gtype, rows, cols)
+    x = g.standard_normal(cols).astype(np.float32)
+    print(f"row length {ggml.NAMES[gtype]} {rows}x{cols}", flush=True)
+    y = gpu_matvec(ctx, w, gtype, rows, cols, x)
+    ref = orc.quant_matvec(w, gtype, x, rows, cols, pool=pool)
+    assert rel_l2(y, ref) <= 3e-6, rel_l2(y, ref)
+
+
+@pytest.mark.parametrize("gtype,cols", [(ggml.Q8_0, 2080), (ggml.Q8_0, 256), (ggml.Q4_K, 768), (ggml.Q6_K, 768)])
+def test_gpu_matvec_any_row_length_nan_inf_small(ctx, gtype, cols):
+    # NaN reaches every output; an infinity gives what the oracle gives;
+    # activations near 2^-90 keep fp32's precision
+    g = np.random.default_rng(cols)
+    rows = 70
+    w = synth.quant_matrix(g, gtype, rows, cols)
+    x = g.standard_normal(cols).astype(np.float32)
+    x[cols // 3] = np.nan
+    assert np.isnan(gpu_matvec(ctx, w, gtype, rows, cols, x)).all()
+    x[cols // 3] = np.inf
+    with np.errstate(all="ignore"):
+        ref = orc.quant_matvec(w, gtype, x, rows, cols)
+    y = gpu_matvec(ctx, w, gtype, rows, cols, x)
+    if gtype == ggml.Q8_0:
+        assert np.array_equal(np.isnan(y), np.isnan(ref)) and np.array_equal(np.isposinf(y), np.isposinf(ref))
+    else:  # inf - inf in the offset term
+        assert not np.isfinite(y).any()
+    x[cols // 3] = 1.0
+    x *= np.float32(2.0 ** -90)
+    ref = orc.quant_matvec(w, gtype, x, rows, cols)
+    assert rel_l2(gpu_matvec(ctx, w, gtype, rows, cols, x).astype(np.float64) * 2.0 ** 90,
+                  ref.astype(np.float64) * 2.0 ** 90) <= 3e-6
+
+
 def test_gpu_config1_dense_ffn_q8_0(ctx):
     c = synth.config1()
     D, F = c["d_model"], c["d_ffn"]
