@@ -744,17 +744,32 @@ int check_router(lt_ctx *ctx, const lt_tensor *router, size_t d_model, uint32_t 
     return LT_OK;
 }
 
-// logits -> ids/w in context buffers (and scores, if non-NULL); x, bias,
-// scores device pointers.
-int router_dev(lt_ctx *ctx, const DevTensor &R, const float *x, const float *bias, uint32_t k, uint32_t flags,
-               float *scores = nullptr, const lt::RouterPrep *prep = nullptr) {
+// Where a call's kernels put the selection: the caller's device arrays, or
+// the context's buffers for an array the caller left out or holds on the host
+// (copy_routing_out takes it from there).  A copy per array behind the
+// kernels cost about 2 us each (router, gate/up and down by ids: 25.9 us with
+// the copies and the router's fences, 20.7 without).
+struct Routing {
+    uint32_t *ids;
+    float *w;
+};
+
+int routing_at(lt_ctx *ctx, uint32_t *ids, float *w, bool host, Routing &r) {
     int rc;
-    if ((rc = ensure(ctx, ctx->logits, R.total_rows * 4)) || (rc = ensure(ctx, ctx->ids, kMaxK * 4)) ||
-        (rc = ensure(ctx, ctx->w, kMaxK * 4)))
-        return rc;
+    if ((rc = ensure(ctx, ctx->ids, kMaxK * 4)) || (rc = ensure(ctx, ctx->w, kMaxK * 4))) return rc;
+    r.ids = ids && !host ? ids : (uint32_t *)ctx->ids.p;
+    r.w = w && !host ? w : (float *)ctx->w.p;
+    return LT_OK;
+}
+
+// logits -> ids / w (and scores, if non-NULL); all device pointers.
+int router_dev(lt_ctx *ctx, const DevTensor &R, const float *x, const float *bias, uint32_t k, uint32_t flags,
+               const Routing &r, float *scores = nullptr, const lt::RouterPrep *prep = nullptr) {
+    int rc;
+    if ((rc = ensure(ctx, ctx->logits, R.total_rows * 4))) return rc;
     float *logits = (float *)ctx->logits.p;
-    hipError_t e = lt::launch_router(R, x, bias, logits, ctx->ticket, k, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u,
-                                     (uint32_t *)ctx->ids.p, (float *)ctx->w.p, scores, ctx->stream, prep);
+    hipError_t e = lt::launch_router(R, x, bias, logits, ctx->ticket, k, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u, r.ids,
+                                     r.w, scores, ctx->stream, prep);
     return launch_rc(ctx, e, "router_topk");
 }
 
@@ -764,10 +779,11 @@ int stage_bias(lt_ctx *ctx, const float *bias, size_t n, bool host, const float 
     return LT_OK;
 }
 
+// The selection to the caller's host arrays (device arrays: the kernels wrote them).
 int copy_routing_out(lt_ctx *ctx, uint32_t k, uint32_t *ids, float *w, bool host) {
-    const hipMemcpyKind kind = host ? hipMemcpyDeviceToHost : hipMemcpyDeviceToDevice;
-    if (ids) LT_HIP(ctx, hipMemcpyAsync(ids, ctx->ids.p, k * 4, kind, ctx->stream));
-    if (w) LT_HIP(ctx, hipMemcpyAsync(w, ctx->w.p, k * 4, kind, ctx->stream));
+    if (!host) return LT_OK;
+    if (ids) LT_HIP(ctx, hipMemcpyAsync(ids, ctx->ids.p, k * 4, hipMemcpyDeviceToHost, ctx->stream));
+    if (w) LT_HIP(ctx, hipMemcpyAsync(w, ctx->w.p, k * 4, hipMemcpyDeviceToHost, ctx->stream));
     return LT_OK;
 }
 
@@ -815,12 +831,12 @@ int gate_up_dev(lt_ctx *ctx, const DevTensor &GU, const float *x, const uint32_t
 }
 
 // gate/up that selects the experts itself from the router logits in
-// ctx->logits and leaves the selection in ctx->ids / ctx->w
+// ctx->logits and leaves the selection in r
 int gate_up_routed_dev(lt_ctx *ctx, const DevTensor &GU, const float *x, uint32_t k, uint32_t norm,
-                       uint32_t d_expert, uint32_t Kd, uint32_t act, float *h) {
+                       uint32_t d_expert, uint32_t Kd, uint32_t act, float *h, const Routing &r) {
     const float *logits = (const float *)ctx->logits.p;
-    uint32_t *ids = (uint32_t *)ctx->ids.p;
-    float *w = (float *)ctx->w.p;
+    uint32_t *ids = r.ids;
+    float *w = r.w;
     if (GU.type == LT_TYPE_Q4_K)
         return launch_rc(ctx,
                          lt::launch_expert_gate_up_q4k_routed(GU, x, logits, k, norm, d_expert, Kd, act, h, ids, w,
@@ -861,7 +877,9 @@ extern "C" int lt_moe_router_topk(lt_ctx *ctx, const lt_tensor *router, const fl
         }
     }
     if ((rc = stage_bias(ctx, bias, R.total_rows, host, &dbias))) return rc;
-    if ((rc = router_dev(ctx, R, dx, dbias, k, flags, dscores))) return rc;
+    Routing r;
+    if ((rc = routing_at(ctx, ids, weights, host, r))) return rc;
+    if ((rc = router_dev(ctx, R, dx, dbias, k, flags, r, dscores))) return rc;
     if ((rc = copy_routing_out(ctx, k, ids, weights, host))) return rc;
     if (host) {
         if (scores)
@@ -986,7 +1004,7 @@ lt::FusedLayer fused_layer(const DevTensor &R, const DevTensor &GU, const DevTen
 // The decode MoE layer on device pointers.
 int moe_dev(lt_ctx *ctx, float *out, const float *x, const DevTensor &R, const float *bias, const DevTensor &GU,
             const DevTensor &D, const lt_tensor *sh_gate, const lt_tensor *sh_up, const lt_tensor *sh_down,
-            uint32_t k, uint32_t d_expert, uint32_t act, uint32_t flags) {
+            uint32_t k, uint32_t d_expert, uint32_t act, uint32_t flags, const Routing &r) {
     int rc;
     const size_t Kd = D.cols;
     // (Q4_K experts, or the APEX formats: Q3_K gate/up, IQ4_NL / Q5_0 / Q5_1
@@ -1013,9 +1031,7 @@ int moe_dev(lt_ctx *ctx, float *out, const float *x, const DevTensor &R, const f
                     return rc;
                 base = (const float *)ctx->shared.p;
             }
-            if ((rc = ensure_fused(ctx)) || (rc = ensure(ctx, ctx->ids, kMaxK * 4)) ||
-                (rc = ensure(ctx, ctx->w, kMaxK * 4)))
-                return rc;
+            if ((rc = ensure_fused(ctx))) return rc;
             ctx->prof.stamps_pending = ctx->prof.stamps != nullptr;
             return launch_rc(ctx,
                              lt::launch_moe_fused(pl,
@@ -1023,8 +1039,8 @@ int moe_dev(lt_ctx *ctx, float *out, const float *x, const DevTensor &R, const f
                                                               k, d_expert, flags),
                                                   bias, x, act, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u, base,
                                                   (flags & LT_MOE_ACCUMULATE) ? 1 : 0,
-                                                  (flags & LT_MOE_DETERMINISTIC) ? 1 : 0, out, (uint32_t *)ctx->ids.p,
-                                                  (float *)ctx->w.p, ctx->fsc, ctx->stream),
+                                                  (flags & LT_MOE_DETERMINISTIC) ? 1 : 0, out, r.ids, r.w, ctx->fsc,
+                                                  ctx->stream),
                              "moe_fused");
         }
     }
@@ -1040,14 +1056,15 @@ int moe_dev(lt_ctx *ctx, float *out, const float *x, const DevTensor &R, const f
     float *h = (float *)ctx->eh.p;
     if (R.total_rows <= kRoutedGateUpMaxExperts) {
         // logits only; each gate/up block selects its expert from them
-        if ((rc = router_dev(ctx, R, x, bias, 0, flags))) return rc;
-        rc = gate_up_routed_dev(ctx, GU, x, k, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u, d_expert, (uint32_t)Kd, act, h);
+        if ((rc = router_dev(ctx, R, x, bias, 0, flags, r))) return rc;
+        rc = gate_up_routed_dev(ctx, GU, x, k, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u, d_expert, (uint32_t)Kd, act, h,
+                                r);
     } else {
-        if ((rc = router_dev(ctx, R, x, bias, k, flags))) return rc;
-        rc = gate_up_dev(ctx, GU, x, (const uint32_t *)ctx->ids.p, k, d_expert, (uint32_t)Kd, act, h);
+        if ((rc = router_dev(ctx, R, x, bias, k, flags, r))) return rc;
+        rc = gate_up_dev(ctx, GU, x, r.ids, k, d_expert, (uint32_t)Kd, act, h);
     }
     if (rc) return rc;
-    return down_dev(ctx, D, h, (const uint32_t *)ctx->ids.p, (const float *)ctx->w.p, k, base,
+    return down_dev(ctx, D, h, r.ids, r.w, k, base,
                     (flags & LT_MOE_ACCUMULATE) ? 1 : 0, nullptr, out);
 }
 
@@ -1085,8 +1102,10 @@ extern "C" int lt_moe_forward(lt_ctx *ctx, float *out, const float *x, const lt_
         return fail(ctx, LT_ERR_INVALID, "x must be 16-byte aligned");
     }
     if ((rc = stage_bias(ctx, router_bias, router->t.total_rows, host, &dbias))) return rc;
+    Routing r;
+    if ((rc = routing_at(ctx, out_ids, out_w, host, r))) return rc;
     rc = moe_dev(ctx, dout, dx, router->t, dbias, gate_up->t, down->t, shared ? sh_gate : nullptr, sh_up, sh_down, k,
-                 d_expert, act, flags);
+                 d_expert, act, flags, r);
     if (rc) return rc;
     if ((rc = copy_routing_out(ctx, k, out_ids, out_w, host))) return rc;
     if (host) {
@@ -1139,17 +1158,14 @@ extern "C" int lt_moe_forward_noalloc(lt_ctx *ctx, float *out, const float *x, c
                     "<= 256 experts, k <= 16, and the grid's room for the shared FFN)",
                     GU.cols, R.total_rows, d_expert, D.cols, k, shared ? ", shared FFN" : "");
     ctx->prof.stamps_pending = ctx->prof.stamps != nullptr;
-    uint32_t *ids_dev = (uint32_t *)(ctx->na_base + lt::kFusedIdsOff);
-    float *w_dev = (float *)(ctx->na_base + lt::kFusedWOff);
+    uint32_t *ids_dev = out_ids ? out_ids : (uint32_t *)(ctx->na_base + lt::kFusedIdsOff);
+    float *w_dev = out_w ? out_w : (float *)(ctx->na_base + lt::kFusedWOff);
     rc = launch_rc(ctx,
                    lt::launch_moe_fused(pl, L, router_bias, x, act, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u, nullptr,
                                         (flags & LT_MOE_ACCUMULATE) ? 1 : 0, (flags & LT_MOE_DETERMINISTIC) ? 1 : 0,
                                         out, ids_dev, w_dev, ctx->na_fsc, ctx->stream),
                    "moe_fused (allocation-free)");
-    if (rc) return rc;
-    if (out_ids) LT_HIP(ctx, hipMemcpyAsync(out_ids, ids_dev, k * 4, hipMemcpyDeviceToDevice, ctx->stream));
-    if (out_w) LT_HIP(ctx, hipMemcpyAsync(out_w, w_dev, k * 4, hipMemcpyDeviceToDevice, ctx->stream));
-    return LT_OK;
+    return rc;
 }
 
 extern "C" int lt_moe_prefill(lt_ctx *ctx, float *out, const float *X, uint32_t T, const lt_tensor *router,
@@ -1404,6 +1420,8 @@ extern "C" int lt_gemma4_moe_block(lt_ctx *ctx, float *x, const float *dense_ffn
         (rc = io_in(ctx, host, ar, post_ffw_norm_2, n, &dp2)) || (rc = io_in(ctx, host, ar, post_ffw_norm, n, &dp)))
         return rc;
     float *xio = const_cast<float *>(dx);
+    Routing r;
+    if ((rc = routing_at(ctx, out_ids, out_w, host, r))) return rc;
     const float inv_sqrt_d = 1.0f / sqrtf((float)n);
     // the whole block in one launch of the single-launch MoE kernel: Q8_0
     // router, Q4_K or APEX experts, the tree order of the norms (LT_NORM_PRECISE
@@ -1417,14 +1435,11 @@ extern "C" int lt_gemma4_moe_block(lt_ctx *ctx, float *x, const float *dense_ffn
         L.gb = &gb;
         const lt::FusedPlan pl = lt::plan_moe_fused(L);
         if (pl.ok && pl.gemma) {
-            if ((rc = ensure_fused(ctx)) || (rc = ensure(ctx, ctx->ids, kMaxK * 4)) ||
-                (rc = ensure(ctx, ctx->w, kMaxK * 4)))
-                return rc;
+            if ((rc = ensure_fused(ctx))) return rc;
             ctx->prof.stamps_pending = ctx->prof.stamps != nullptr;
             rc = launch_rc(ctx,
                            lt::launch_moe_fused(pl, L, nullptr, dx, act, (flags & LT_MOE_NORM_TOPK) ? 1u : 0u, nullptr,
-                                                0, 0, moe, (uint32_t *)ctx->ids.p, (float *)ctx->w.p, ctx->fsc,
-                                                ctx->stream),
+                                                0, 0, moe, r.ids, r.w, ctx->fsc, ctx->stream),
                            "gemma4_block_fused");
             if (rc) return rc;
             if ((rc = copy_routing_out(ctx, k, out_ids, out_w, host))) return rc;
@@ -1450,15 +1465,14 @@ extern "C" int lt_gemma4_moe_block(lt_ctx *ctx, float *x, const float *dense_ffn
     float *h = (float *)ctx->eh.p;
     const uint32_t norm = (flags & LT_MOE_NORM_TOPK) ? 1u : 0u;
     if (E <= kRoutedGateUpMaxExperts) {
-        if ((rc = router_dev(ctx, R, rin, nullptr, 0, flags, nullptr, fuse_prep ? &prep : nullptr))) return rc;
-        rc = gate_up_routed_dev(ctx, GU, moe_in, k, norm, d_expert, (uint32_t)Kd, act, h);
+        if ((rc = router_dev(ctx, R, rin, nullptr, 0, flags, r, nullptr, fuse_prep ? &prep : nullptr))) return rc;
+        rc = gate_up_routed_dev(ctx, GU, moe_in, k, norm, d_expert, (uint32_t)Kd, act, h, r);
     } else {
-        if ((rc = router_dev(ctx, R, rin, nullptr, k, flags, nullptr, fuse_prep ? &prep : nullptr))) return rc;
-        rc = gate_up_dev(ctx, GU, moe_in, (const uint32_t *)ctx->ids.p, k, d_expert, (uint32_t)Kd, act, h);
+        if ((rc = router_dev(ctx, R, rin, nullptr, k, flags, r, nullptr, fuse_prep ? &prep : nullptr))) return rc;
+        rc = gate_up_dev(ctx, GU, moe_in, r.ids, k, d_expert, (uint32_t)Kd, act, h);
     }
     if (rc) return rc;
-    if ((rc = down_dev(ctx, D, h, (const uint32_t *)ctx->ids.p, (const float *)ctx->w.p, k, nullptr, 0, dds, moe)))
-        return rc;
+    if ((rc = down_dev(ctx, D, h, r.ids, r.w, k, nullptr, 0, dds, moe))) return rc;
     // 482-497: post_ffw_norm_2, + dense FFN, post_ffw_norm, residual, layer_output_scale
     if ((rc = norm_run(ctx, 3, moe, dd, dp, dp2, xio, nullptr, 1, (uint32_t)n, eps, layer_output_scale, flags)))
         return rc;

@@ -23,7 +23,7 @@ namespace lt {
 namespace {
 
 struct TopkArgs {
-    unsigned *ticket;  // zero-initialised; wraps back to 0 after each launch
+    unsigned *ticket;  // zero-initialised; the last block puts it back to 0
     int k;             // 0: logits only
     int norm;
     uint32_t *ids;
@@ -31,26 +31,38 @@ struct TopkArgs {
     float *scores;
 };
 
-// After this block's logits are stored: the last block to arrive runs the
-// top-k.  Must be called by every thread of the block.
+// Logits go out with agent-scope stores (past the XCD's own L2), so that the
+// last block can read the other blocks' without a cache write-back: a release
+// fence there writes back the whole L2 (128 rows of 2,048: the launch took
+// 8.2 us with fences, 5.2 without, both with the top-k).
+__device__ __forceinline__ void put_logit(float *p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// After this block's logits are stored (put_logit): the last block to arrive
+// runs the top-k.  Must be called by every thread of the block.  A thread's
+// stores are acknowledged before its block takes a ticket, so the block that
+// draws the last ticket reads every logit.
 __device__ __forceinline__ void last_block_topk(const float *logits, int n, const TopkArgs &a) {
     if (a.k == 0) return;
     __shared__ int is_last;
-    __threadfence();  // release this block's logits
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __syncthreads();
-    if (threadIdx.x == 0) is_last = atomicInc(a.ticket, gridDim.x - 1) == gridDim.x - 1;
+    if (threadIdx.x == 0) {
+        is_last = __hip_atomic_fetch_add(a.ticket, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == gridDim.x - 1;
+        if (is_last) __hip_atomic_store(a.ticket, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
     __syncthreads();
     if (is_last && threadIdx.x < 64) {
-        __threadfence();  // acquire the other blocks' logits
         const int lane = threadIdx.x;
         if (n <= 64)
-            topk_softmax_wave<1>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
+            topk_softmax_wave<1, true>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
         else if (n <= 128)
-            topk_softmax_wave<2>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
+            topk_softmax_wave<2, true>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
         else if (n <= 256)
-            topk_softmax_wave<4>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
+            topk_softmax_wave<4, true>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
         else
-            topk_softmax_wave<16>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
+            topk_softmax_wave<16, true>(logits, n, a.k, a.norm, a.ids, a.w, a.scores, lane);
     }
 }
 
@@ -113,7 +125,91 @@ __global__ void __launch_bounds__(64) k_router_f32(const float *__restrict__ W, 
             sum = sum + p;
         }
         if (bias) sum = sum + bias[row];
-        logits[row] = sum;
+        put_logit(logits + row, sum);
+    }
+    last_block_topk(logits, rows, ta);
+}
+
+// The same logits for rows of a multiple of 256 elements and x on a 16-byte
+// boundary, two rows a block: wavefront w takes chains 16 (w & 1) + [0, 16)
+// of row 2 blockIdx.x + (w >> 1), so that a row is on its way in two
+// wavefronts' 16-byte loads (lane L of load q: stride 16 q + L / 4, chains
+// 4 (L & 3) + [0, 4) of the wavefront's).  The products of a load pass
+// through LDS to the chain lanes (chain c = lane & 15), which add them stride
+// by stride; (acc0 + acc1) is formed in each wavefront, (acc2 + acc3) crosses
+// to the row's first one, which finishes the ordered sum: dotf32's rounded
+// operations in its order.  Loads go in batches of 4 (2,048 elements), the
+// next batch's before this one's products are added.  Bound by the launch,
+// one round trip to memory and the chain of adds (64 a row of 2,048):
+// 128 x 2,048 4.7 -> 3.35 us, 64 x 1,024 3.8 -> 2.9 against k_router_f32.
+__global__ void __launch_bounds__(256) k_router_f32_pair(const float *__restrict__ W, const float *__restrict__ x,
+                                                         const float *__restrict__ bias, float *__restrict__ logits,
+                                                         int rows, int cols, TopkArgs ta) {
+#pragma clang fp contract(off)
+    __shared__ __attribute__((aligned(16))) float prod_all[4][512];  // per wavefront: two [16][16] buffers
+    __shared__ float xch[2][8];
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int nit = cols >> 5, h = wave & 1, rl = wave >> 1, row = 2 * blockIdx.x + rl;
+    const bool valid = row < rows;
+    const float *wr = W + (size_t)(valid ? row : 0) * cols;
+    float *prod = prod_all[wave];
+    float4 wv[2][4], xv[2][4];
+    auto load_batch = [&](int b, int qb) {  // unconditional: strides clamped
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int it = min(16 * (qb + q) + (lane >> 2), nit - 1);
+            const int e = 32 * it + 16 * h + 4 * (lane & 3);
+            wv[b][q] = ldg16f(wr + e);
+            xv[b][q] = ldg16f(x + e);
+        }
+    };
+    load_batch(0, 0);
+    const float bv = bias ? bias[valid ? row : 0] : 0.0f;
+    float acc = 0.0f;
+    auto add_batch = [&](int b, int qb) {
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            if (16 * (qb + q) < nit) {
+                float4 pr;
+                pr.x = wv[b][q].x * xv[b][q].x;
+                pr.y = wv[b][q].y * xv[b][q].y;
+                pr.z = wv[b][q].z * xv[b][q].z;
+                pr.w = wv[b][q].w * xv[b][q].w;
+                float *buf = prod + (q & 1) * 256;
+                *reinterpret_cast<float4 *>(buf + 4 * lane) = pr;
+                __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+                __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+                const int n = nit - 16 * (qb + q);  // 8 (the rest is not added) or 16 and more
+                float v[16];
+#pragma unroll
+                for (int u = 0; u < 16; u++) v[u] = buf[u * 16 + (lane & 15)];
+#pragma unroll
+                for (int u0 = 0; u0 < 16; u0 += 8)
+                    if (u0 < n)
+#pragma unroll
+                        for (int u = 0; u < 8; u++) acc = acc + v[u0 + u];
+            }
+        }
+    };
+    for (int qb = 0; 16 * qb < nit; qb += 8) {
+        if (16 * (qb + 4) < nit) load_batch(1, qb + 4);
+        add_batch(0, qb);
+        if (16 * (qb + 4) < nit) {
+            if (16 * (qb + 8) < nit) load_batch(0, qb + 8);
+            add_batch(1, qb + 4);
+        }
+    }
+    const float s2 = acc + dpp<0x128>(acc);  // lanes l < 8: chains 16 h + l and 16 h + l + 8
+    if (h == 1 && lane < 8) xch[rl][lane] = s2;
+    __syncthreads();
+    if (h == 0) {
+        const float a8 = s2 + xch[rl][lane & 7];
+        float sum = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a8), 0));
+#pragma unroll
+        for (int l = 1; l < 8; l++) sum = sum + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(a8), l));
+        if (bias) sum = sum + bv;
+        if (lane == 0 && valid) put_logit(logits + row, sum);
     }
     last_block_topk(logits, rows, ta);
 }
@@ -240,7 +336,7 @@ __global__ void __launch_bounds__(128) k_router_q8_0(const int8_t *__restrict__ 
         float total = 0.0f;
         for (int b = 0; b < nb; b++) total = total + term[b];
         if (bias) total = total + bias[row];
-        logits[row] = total;
+        put_logit(logits + row, total);
     }
     last_block_topk(logits, rows, ta);
 }
@@ -254,8 +350,15 @@ hipError_t launch_router(const DevTensor &R, const float *x, const float *bias, 
     const int rows = (int)R.total_rows;
     if (R.type == 0) {  // F32
         const int cols = (int)R.cols;
-        hipLaunchKernelGGL(k_router_f32<64>, dim3((rows + 1) / 2), dim3(64), 0, s, (const float *)R.p0, x, bias,
-                           logits, rows, cols, ta);
+        // A router's few rows (other row lengths have a tail in dotf32's
+        // order, and 4-byte loads take any x).  Large matrices fill the chip
+        // either way: 32,000 x 2,048 takes 43.5 us in pairs, 42.6 without.
+        if (rows <= 1024 && cols % 256 == 0 && ((uintptr_t)x & 15u) == 0)
+            hipLaunchKernelGGL(k_router_f32_pair, dim3((rows + 1) / 2), dim3(256), 0, s, (const float *)R.p0, x, bias,
+                               logits, rows, cols, ta);
+        else
+            hipLaunchKernelGGL(k_router_f32<64>, dim3((rows + 1) / 2), dim3(64), 0, s, (const float *)R.p0, x, bias,
+                               logits, rows, cols, ta);
     } else {  // Q8_0
         const int nb = (int)R.blocks_per_row;
         hipLaunchKernelGGL(k_router_q8_0, dim3(rows), dim3(128), nb * sizeof(float), s, (const int8_t *)R.p0,

@@ -44,14 +44,18 @@ __device__ void topk_softmax_regs(const float (&vin)[PER], int n, int k, int nor
                                   uint32_t (&key)[PER], int &my_i_out, float &my_p_out, int lane);
 
 // Loads lane + 64*j (j < PER) of logits[0..n) and runs topk_softmax_regs.
-template <int PER>
+// AGENT: the logits come from other blocks of the same launch (agent-scope
+// stores), so they are read at that scope.
+template <int PER, bool AGENT = false>
 __device__ void topk_softmax_wave(const float *logits, int n, int k, int norm, uint32_t *ids, float *w,
                                   float *scores, int lane) {
     float v[PER];
 #pragma unroll
     for (int j = 0; j < PER; j++) {
         const int idx = lane + 64 * j;
-        v[j] = idx < n ? logits[idx] : -INFINITY;
+        v[j] = -INFINITY;
+        if (idx < n)
+            v[j] = AGENT ? __hip_atomic_load(logits + idx, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : logits[idx];
     }
     uint32_t key[PER];
     int my_i;
@@ -62,7 +66,7 @@ __device__ void topk_softmax_wave(const float *logits, int n, int k, int norm, u
         for (int j = 0; j < PER; j++) {
             const int idx = lane + 64 * j;
             if (idx < n) {
-                float val = logits[idx];
+                float val = v[j];
                 if (key[j] == 0)  // selected (cleared)
                     for (int r = 0; r < k; r++)
                         if (__builtin_amdgcn_readlane(my_i, r) == idx)

@@ -14,7 +14,7 @@ import pytest
 
 import llmtoy_amd as lt
 import pyoracle as orc
-from llmtoy_amd import ggml, synth
+from llmtoy_amd import ggml, hip, synth
 from llmtoy_amd.lib import DeviceError, InvalidError, UnsupportedError
 
 pytestmark = pytest.mark.gpu
@@ -416,6 +416,38 @@ def test_gpu_config3_router_logits_bit_exact(ctx, cfg3):
         rest = np.setdiff1d(np.arange(w.n_experts), ids)
         assert np.array_equal(scores[rest].view(np.uint32), logits[rest].view(np.uint32))
         assert ids.tolist() == orc.topk_softmax_stats(logits, 8)[0].tolist()
+
+
+@pytest.mark.parametrize("E,D", [(1, 256), (3, 512), (63, 2048), (65, 2304), (130, 4096), (257, 6400), (1024, 256)])
+def test_gpu_router_row_pairs_bit_exact(ctx, E, D):
+    # two rows a block, loads in batches of 2,048 elements: odd row counts and
+    # rows of half, one, and several batches, logits bit for bit, and the
+    # same with x off the 16-byte boundary (the 4-byte path)
+    g = np.random.default_rng(E + D)
+    W = (g.standard_normal((E, D)) * 0.02).astype(np.float32)
+    x = g.standard_normal(D).astype(np.float32)
+    k = min(E, 8)
+    router = ctx.upload(W, ggml.F32, E, D)
+    ref = orc.quant_matvec(W, orc.F32, x, E, D)
+    want, top, total = orc.topk_softmax_stats(ref, k)
+    prob = np.exp(ref[want] - top) / total
+    xd = hip.DeviceArray((D + 1,))
+    for off in (0, 1):
+        buf = np.zeros(D + 1, np.float32)
+        buf[off:off + D] = x
+        hip.check(hip.hip().hipMemcpy(xd.ptr, buf.ctypes.data, buf.nbytes, hip.H2D))
+        ids, w, scores = hip.DeviceArray((k,), np.uint32), hip.DeviceArray((k,)), hip.DeviceArray((E,))
+        ctx.router_topk(router, hip.DeviceView(xd.ptr + 4 * off, (D,), np.float32), k, ids, w, scores=scores)
+        ctx.sync()
+        got = ids.numpy()
+        rest = np.setdiff1d(np.arange(E), got)
+        assert got.tolist() == want.tolist()
+        assert np.array_equal(scores.numpy()[rest].view(np.uint32), ref[rest].view(np.uint32))
+        assert np.allclose(w.numpy(), prob, rtol=1e-5, atol=0)
+        for d in (ids, w, scores):
+            d.free()
+    xd.free()
+    router.free()
 
 
 def test_gpu_config3_expert_stages_compose(ctx, cfg3, pool):
