@@ -21,75 +21,11 @@
 #include "lt_internal.h"
 #include "lt_topk.h"
 #include "lt_limbs.h"
+#include "lt_rows.h"
 
 namespace lt {
 
 namespace {
-
-// x values of chunk cc of super-block sb: 16 low-nibble partners and 16
-// high-nibble partners.
-struct XChunk {
-    float lo[16];
-    float hi[16];
-    float slo, shi;  // sums, for the min term
-};
-
-__device__ __forceinline__ void load_xchunk(const float *xs, int sb, int cc, XChunk &xc) {
-    const float *p = xs + sb * 256 + 64 * (cc >> 1) + 16 * (cc & 1);
-#pragma unroll
-    for (int t = 0; t < 16; t += 4) {
-        float4 a = *reinterpret_cast<const float4 *>(p + t);
-        float4 b = *reinterpret_cast<const float4 *>(p + 32 + t);
-        xc.lo[t] = a.x; xc.lo[t + 1] = a.y; xc.lo[t + 2] = a.z; xc.lo[t + 3] = a.w;
-        xc.hi[t] = b.x; xc.hi[t + 1] = b.y; xc.hi[t + 2] = b.z; xc.hi[t + 3] = b.w;
-    }
-}
-
-// The x sums used by the min term; kept apart from load_xchunk so that the
-// adds can be placed after the weight loads are issued.
-__device__ __forceinline__ void sum_xchunk(XChunk &xc) {
-    float slo = 0.f, shi = 0.f;
-#pragma unroll
-    for (int t = 0; t < 16; t += 4) {
-        slo += (xc.lo[t] + xc.lo[t + 1]) + (xc.lo[t + 2] + xc.lo[t + 3]);
-        shi += (xc.hi[t] + xc.hi[t + 1]) + (xc.hi[t + 2] + xc.hi[t + 3]);
-    }
-    xc.slo = slo;
-    xc.shi = shi;
-}
-
-// Dot of one 16-byte qs chunk with its x values.
-__device__ __forceinline__ float q4k_chunk_dot(uint4 hdr, uint4 q, int cc, const XChunk &xc) {
-    const float d = f16_bits_to_f32(hdr.x);
-    const float dmin = f16_bits_to_f32(hdr.x >> 16);
-    // get_scale_min_k4 for the sub-block pair (2p, 2p+1) of this chunk, both
-    // fields at once: the pair's bytes sit at byte offset 2*(p&1) of the
-    // scale words (hdr.y = scales[0..3], hdr.z = [4..7], hdr.w = [8..11]).
-    const int p = cc >> 1;
-    const int sh = (p & 1) * 16;
-    const uint32_t ys = hdr.y >> sh, zs = hdr.z >> sh, ws = hdr.w >> sh;
-    const uint32_t scp = opaque(p < 2 ? (ys & 0x3f3fu) : ((ws & 0x0f0fu) | ((ys >> 2) & 0x3030u)));
-    const uint32_t mnp = opaque(p < 2 ? (zs & 0x3f3fu) : (((ws >> 4) & 0x0f0fu) | ((zs >> 2) & 0x3030u)));
-    const float sc0 = (float)(scp & 0xffu), sc1 = (float)((scp >> 8) & 0xffu);
-    const float mn0 = (float)(mnp & 0xffu), mn1 = (float)((mnp >> 8) & 0xffu);
-    const uint32_t w[4] = {q.x, q.y, q.z, q.w};
-    float dl0 = 0.f, dl1 = 0.f, dh0 = 0.f, dh1 = 0.f;
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const uint32_t lo = opaque(w[t] & 0x0f0f0f0fu);
-        const uint32_t hi = opaque((w[t] >> 4) & 0x0f0f0f0fu);
-        dl0 = fmaf((float)(lo & 0xffu), xc.lo[4 * t + 0], dl0);
-        dl1 = fmaf((float)((lo >> 8) & 0xffu), xc.lo[4 * t + 1], dl1);
-        dl0 = fmaf((float)((lo >> 16) & 0xffu), xc.lo[4 * t + 2], dl0);
-        dl1 = fmaf((float)(lo >> 24), xc.lo[4 * t + 3], dl1);
-        dh0 = fmaf((float)(hi & 0xffu), xc.hi[4 * t + 0], dh0);
-        dh1 = fmaf((float)((hi >> 8) & 0xffu), xc.hi[4 * t + 1], dh1);
-        dh0 = fmaf((float)((hi >> 16) & 0xffu), xc.hi[4 * t + 2], dh0);
-        dh1 = fmaf((float)(hi >> 24), xc.hi[4 * t + 3], dh1);
-    }
-    const float dl = dl0 + dl1, dh = dh0 + dh1;
-    return ((d * sc0) * dl - (dmin * mn0) * xc.slo) + ((d * sc1) * dh - (dmin * mn1) * xc.shi);
-}
 
 // The limbs of one chunk's activations (lt_limbs.h): group 0 = the 16
 // low-nibble partners, group 1 = the 16 high-nibble partners.
@@ -479,73 +415,85 @@ hipError_t launch_expert_gate_up_q4k_routed(const DevTensor &GU, const float *x,
 //   out[i] = base[i] + sum_{s in slot order} w[s] * (D_{ids[s]} row i) . h[s]
 // (w[s] times dscale[ids[s]] when a per-expert down scale is given)
 // (base = previous out with accumulate, the shared-FFN output, or 0).
-// Block: NW = min(nsb, 4) waves x RD output rows.  Wave w handles
-// super-blocks w, w+NW, ... of the K = down_cols dimension; lane = (slot
-// within an 8-slot pass, chunk cc), so one load instruction covers the same
-// super-block of 8 experts (8 contiguous 128-byte runs).  Per-(row, slot,
-// super-block) partial sums go through LDS and are combined in a fixed
-// order, so the result does not depend on scheduling.
-template <int RD>
-__global__ void __launch_bounds__(256) k_expert_down_q4k(const uint8_t *__restrict__ hdr,
-                                                         const uint8_t *__restrict__ qs,
-                                                         const float *__restrict__ h,
-                                                         const uint32_t *__restrict__ ids,
-                                                         const float *__restrict__ wts, int k, int n_experts,
-                                                         int rows_per_expert, int nsb, const float *base,
-                                                         int accumulate, const float *dscale, float *out) {
-    __shared__ float part[RD][16][16];  // [row][slot][super-block]
-    const int NW = blockDim.x / kWave;
-    const int w = threadIdx.x / kWave, lane = threadIdx.x % kWave;
-    const int sl = lane >> 3, cc = lane & 7;
-    const int row0 = blockIdx.x * RD;
-    const int K = nsb * 256;
-    for (int pass = 0; pass * 8 < k; pass++) {
-        const int s = pass * 8 + sl;
-        const bool active = s < k;
-        const uint32_t e = active ? ids[s] : 0u;
-        const bool valid = active && e < (uint32_t)n_experts;
-        const float *hs = h + (size_t)(valid ? s : 0) * K;
-        for (int sb = w; sb < nsb; sb += NW) {
-            XChunk xc;
-            load_xchunk(hs, sb, cc, xc);
-            uint4 hv[RD], qv[RD];
+// An output row is P = k U work units of 64 weights (slot s, unit u of the
+// slot's expert).  A thread keeps one of these positions, with its slot's 64
+// activations in registers (lt_rows.h), and a workgroup of RP = threads / P
+// rows side by side walks the output rows, the next pass's weights on their
+// way while the partial sums of this one meet in LDS: a slot's U units are
+// added in order, then the slots in order, so the result does not depend on
+// scheduling.  Two rows per workgroup, with the activations read again by every
+// workgroup and a 16-byte header by every lane, took 7.8 us for 8 slots of
+// 2,048 x 768; this takes 6.5 (kernel trace, medians), 0.3 us of it saved by
+// loading ids, weights and old outputs at the start.  Bound by the launch and
+// the chain load -> dot -> two barriers.  h goes through LDS (quad by quad, no
+// bank conflicts) up to 64 KB, longer rows read it as they are.
+template <bool STAGED>
+__global__ void __launch_bounds__(1024) k_expert_down_q4k(DevTensor W, const float *__restrict__ h,
+                                                          const uint32_t *__restrict__ ids,
+                                                          const float *__restrict__ wts, int k, int U, int RP,
+                                                          const float *base, int accumulate, const float *dscale,
+                                                          float *out) {
+    extern __shared__ __attribute__((aligned(16))) float lds[];
+    float4 *hs = reinterpret_cast<float4 *>(lds);  // [16][P] quads (STAGED)
+    const int tid = threadIdx.x, NT = blockDim.x, P = k * U;
+    float *part = lds + (STAGED ? 64 * P : 0), *slot = part + NT;  // [RP][P], then [RP][k]
+    __shared__ float s_w[16];                                      // the slots' combine weights
+    const int r = min(tid / P, RP - 1), pos = tid % P, s = pos / U, u = pos % U;
+    const int rows = (int)W.rows, npass = (rows + RP - 1) / RP;
+    const uint32_t e = ids[s];
+    const bool valid = e < (uint32_t)W.n_experts;
+    const size_t e0 = (size_t)(valid ? e : 0u) * rows;
+    float4 hv[3];
+    const int nq = 16 * P;  // quads of h
+    if (STAGED) {
 #pragma unroll
-            for (int r = 0; r < RD; r++) {
-                const int row = row0 + r;
-                if (valid && row < rows_per_expert) {
-                    const size_t blk = ((size_t)e * rows_per_expert + row) * nsb + sb;
-                    hv[r] = ldg16(hdr + blk * 16);
-                    qv[r] = ldg16(qs + blk * 128 + cc * 16);
-                }
-            }
-            sum_xchunk(xc);
-            float v[RD];
-#pragma unroll
-            for (int r = 0; r < RD; r++)
-                v[r] = (valid && row0 + r < rows_per_expert) ? q4k_chunk_dot(hv[r], qv[r], cc, xc) : 0.f;
-            // lane (slot, cc) receives the 8-lane total of row cc * RD / 8
-            const float t = group8_sum_transposed<RD>(v, lane);
-            constexpr int SPLIT = 8 / RD;  // lanes per row after the reduction
-            if (active && cc % SPLIT == 0) part[cc / SPLIT][s][sb] = t;
-        }
+        for (int i = 0; i < 3; i++) hv[i] = ldg16f(h + 4 * min(tid + i * NT, nq - 1));
     }
-    __syncthreads();
-    if (threadIdx.x < RD) {
-        const int r = threadIdx.x, row = row0 + r;
-        if (row < rows_per_expert) {
-            float acc = accumulate ? out[row] : 0.f;
-            for (int s = 0; s < k; s++) {
-                float t = part[r][s][0];
-                for (int b = 1; b < nsb; b++) t += part[r][s][b];
-                const uint32_t e = ids[s];
-                if (e < (uint32_t)n_experts) {
-                    // expert_scale = down_exps_scale[e] * w (gemma4/forward.zig:477)
-                    const float ws = dscale ? dscale[e] * wts[s] : wts[s];
-                    acc += ws * t;
-                }
-            }
-            if (base) acc = base[row] + acc;
-            out[row] = acc;
+    asm volatile("" ::: "memory");
+    FmtQ4_K::Regs w;
+    auto ld = [&](int ps) { FmtQ4_K::load(w, W, (e0 + min(ps * RP + r, rows - 1)) * U + u, 0); };
+    int ps = blockIdx.x;
+    ld(ps);
+    float ws = 0.f;
+    if (tid < k) {
+        const uint32_t eq = ids[tid];
+        // expert_scale = down_exps_scale[e] * w (gemma4/forward.zig:477)
+        if (eq < (uint32_t)W.n_experts) ws = dscale ? dscale[eq] * wts[tid] : wts[tid];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    FmtQ4_K::X x;
+    if (STAGED) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            const int f = min(tid + i * NT, nq - 1);
+            hs[(f & 15) * P + (f >> 4)] = hv[i];
+        }
+        for (int f = tid + 3 * NT; f < nq; f += NT) hs[(f & 15) * P + (f >> 4)] = ldg16f(h + 4 * f);
+        __syncthreads();
+        FmtQ4_K::load_acts(x, hs + pos, P);
+    } else {
+        FmtQ4_K::load_acts(x, reinterpret_cast<const float4 *>(h) + 16 * pos, 1);
+    }
+    if (tid < k) s_w[tid] = ws;  // (read two barriers on)
+    for (; ps < npass; ps += gridDim.x) {
+        const int row = ps * RP + tid;
+        const bool mine = tid < RP && row < rows;
+        const float old = mine && accumulate ? out[row] : 0.f, start = mine && base ? base[row] : 0.f;
+        const float t = FmtQ4_K::dot(w, u & 3, x);
+        if (ps + (int)gridDim.x < npass) ld(ps + gridDim.x);
+        part[tid] = valid ? t : 0.f;  // (an id out of range: the slot adds nothing)
+        __syncthreads();
+        if (tid < RP * k) {  // (row, slot): the slot's units in order
+            const float *p = part + tid * U;
+            float sum = p[0];
+            for (int v = 1; v < U; v++) sum += p[v];
+            slot[tid] = sum;
+        }
+        __syncthreads();
+        if (mine) {
+            float acc = old;
+            for (int q = 0; q < k; q++) acc += s_w[q] * slot[tid * k + q];
+            out[row] = base ? start + acc : acc;
         }
     }
 }
@@ -553,13 +501,29 @@ __global__ void __launch_bounds__(256) k_expert_down_q4k(const uint8_t *__restri
 hipError_t launch_expert_down_q4k(const DevTensor &D, const float *h, const uint32_t *ids, const float *w,
                                   uint32_t k, const float *base, int accumulate, float *out, hipStream_t s,
                                   const float *dscale) {
-    constexpr int RD = 2;  // 2 rows per block: 7.5 -> 6.5 us against 8 rows (config 3)
-    const int nsb = (int)D.blocks_per_row;  // <= 16, k <= 16: checked by the API layer
-    const int nw = nsb < 4 ? nsb : 4;
-    const int rows = (int)D.rows;
-    dim3 grid((rows + RD - 1) / RD);
-    hipLaunchKernelGGL((k_expert_down_q4k<RD>), grid, dim3(64 * nw), 0, s, D.p0, D.p1, h, ids, w, (int)k,
-                       (int)D.n_experts, rows, nsb, base, accumulate, dscale, out);
+    const int U = 4 * (int)D.blocks_per_row, P = (int)k * U;  // U <= 64, k <= 16: checked by the API layer
+    // the largest workgroup of up to 512 threads (1,024 for longer rows) that
+    // leaves the fewest lanes idle
+    int nt = 1024;
+    if (P <= 512) {
+        double best = 0;
+        for (int t = 512; t >= 128 && t >= P; t -= 64) {
+            const double used = (double)(t / P * P) / t;
+            if (used > best * 1.01) {
+                best = used;
+                nt = t;
+            }
+        }
+    }
+    const int RP = nt / P, npass = ((int)D.rows + RP - 1) / RP;
+    const int grid = npass < 256 * (1024 / nt) ? npass : 256 * (1024 / nt);
+    const size_t red = ((size_t)nt + (size_t)RP * k) * sizeof(float), stage = (size_t)P * 256;
+    if (stage <= 65536)
+        hipLaunchKernelGGL(k_expert_down_q4k<true>, dim3(grid), dim3(nt), stage + red, s, D, h, ids, w, (int)k, U, RP,
+                           base, accumulate, dscale, out);
+    else
+        hipLaunchKernelGGL(k_expert_down_q4k<false>, dim3(grid), dim3(nt), red, s, D, h, ids, w, (int)k, U, RP, base,
+                           accumulate, dscale, out);
     return hipGetLastError();
 }
 

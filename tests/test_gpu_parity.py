@@ -466,6 +466,47 @@ def test_gpu_config3_expert_stages_compose(ctx, cfg3, pool):
     assert rel_l2(out, ref) <= REL_L2
 
 
+@pytest.mark.parametrize("E,D,Kd,k", [
+    (4, 1, 256, 1), (4, 70, 256, 3),    # 4 and 12 positions a row; fewer rows than a pass
+    (8, 257, 768, 8), (8, 1000, 1024, 5),
+    (8, 300, 4096, 16),                 # 1,024 positions: one row a pass, h not staged
+    (8, 4100, 1280, 9)])                # several passes a workgroup
+def test_gpu_expert_down_positions(ctx, E, D, Kd, k):
+    # out = w . (D h) against the oracle's rows in fp32 (products and sums of
+    # Kd terms rounded to 2^-24: 3e-6 covers both sides), with repeated and
+    # out-of-range ids (those add nothing), accumulating on out
+    g = np.random.default_rng(D + Kd)
+    dm = synth.q4k_matrix(g, E * D, Kd)
+    down = ctx.upload(dm, ggml.Q4_K, D, Kd, E)
+    ids = g.integers(0, E, k).astype(np.uint32)
+    if k > 2:
+        ids[1] = ids[0]
+    w = g.random(k).astype(np.float32)
+    h = g.standard_normal((k, Kd)).astype(np.float32)
+    out0 = g.standard_normal(D).astype(np.float32)
+    ref = out0.astype(np.float64)
+    bad = k > 4
+    idev = ids.copy()
+    if bad:
+        idev[3] = E + 7
+    for s in range(k):
+        if bad and s == 3:
+            continue
+        ref += w[s] * orc.quant_matvec(dm[ids[s] * D:(ids[s] + 1) * D], ggml.Q4_K, h[s], D, Kd).astype(np.float64)
+    dev = [hip.DeviceArray.from_numpy(a) for a in (h, idev, w, out0)]
+    ctx.expert_down_id(down, dev[0], dev[1], dev[2], k, dev[3], accumulate=True)
+    ctx.sync()
+    first = dev[3].numpy()
+    assert rel_l2(first, ref) <= 3e-6, rel_l2(first, ref)
+    hip.check(hip.hip().hipMemcpy(dev[3].ptr, out0.ctypes.data, out0.nbytes, hip.H2D))
+    ctx.expert_down_id(down, dev[0], dev[1], dev[2], k, dev[3], accumulate=True)
+    ctx.sync()
+    assert np.array_equal(first.view(np.uint32), dev[3].numpy().view(np.uint32))
+    for d in dev:
+        d.free()
+    down.free()
+
+
 def test_gpu_config4_gemma_like(ctx, pool):
     c = synth.config4()
     w = c["weights"]
