@@ -6,23 +6,24 @@
 //      and per-token softmax / top-k (lt_router.hip);
 //   2. dispatch: one block counts tokens per expert, lays out per-expert
 //      row ranges ("sorted rows"), cuts each range into chunks of at most
-//      MC = 128 rows, and places the (token, slot) assignments into them in
+//      MC = 64 rows, and places the (token, slot) assignments into them in
 //      assignment order (a stable counting sort);
 //      X is converted to f16 once (by the router kernel, or
 //      k_prefill_x_f16), each row t divided by r_t = 2^e, a power of two
 //      that puts its largest element in [1, 2);
-//   3. grouped gate/up GEMM: one block per (chunk, 64 output columns); its
-//      128 weight rows (64 gate + 64 up) are dequantised from Q4_K to f16
-//      in LDS once per K stage and shared by the chunk's 4 token tiles (one
-//      32-row tile per wavefront, v_mfma_f32_32x32x16_f16, fp32
-//      accumulation); gate and up of an output column sit in the same
-//      wavefront, so the epilogue h = act(gate) * up needs no exchange; it
-//      stores H = h / r_t^2 (f16), which |act(g)| <= |g| bounds by the
-//      scaled row's products whatever X's magnitude (a value still past
-//      f16's range saturates at +-65504 and is counted: the call then
-//      reports LT_ERR_DEVICE);
+//   3. grouped gate/up GEMM: one block per (chunk, 64 output columns), a
+//      wavefront of it per 16 columns: its 32 weight rows (16 gate + the
+//      matching 16 up) are dequantised from Q4_K to f16 in registers, as the
+//      B operand of v_mfma_f32_32x32x16_f16 (fp32 accumulation), and meet the
+//      chunk's one or two 32-row token tiles, which the block shares through
+//      LDS.  Gate and up of an output column sit in the same wavefront, so
+//      the epilogue h = act(gate) * up exchanges values between two halves
+//      of a row only; it stores H = h / r_t^2 (f16), which |act(g)| <= |g|
+//      bounds by the scaled row's products whatever X's magnitude (a value
+//      still past f16's range saturates at +-65504 and is counted: the call
+//      then reports LT_ERR_DEVICE);
 //   4. grouped down GEMM: one block per (chunk, 128 output rows), the same
-//      scheme with H as the A operand -> Y (fp32, sorted rows);
+//      scheme with H as the token operand -> Y (fp32, sorted rows);
 //   5. combine: out[t] = r_t^2 * sum over slots in slot order of w[t][s] *
 //      Y[pos] (r_t^2 exact).
 // Steps 3 and 4 run as one launch when blocks with equal index % 8 share an
@@ -30,14 +31,25 @@
 // blocks through that XCD's L2), else as two.  Chunks of a single token
 // skip the tiles: their blocks stream the weights against int8 limbs of the
 // token like the decode kernels (gate_up_tiny, down_tiny).
-// Both GEMMs run a software pipeline over K stages of 128 (half a Q4_K
-// super-block): weight loads are issued two stages ahead into registers,
-// A fragments one stage ahead, the dequantised tile is double-buffered in
-// LDS, and each stage ends in one barrier.
-// A row's result depends on its chunk only through the chunk's token tiles
-// (they pick the K split of the GEMMs, and with it the order of the fp32
-// sums), and the stable placement gives every row the same chunk on every
-// call, so the output is bit-identical run to run.
+// Both GEMMs run over K stages of 64 (a pair of Q4_K sub-blocks): weights
+// are requested a super-block ahead, tokens two stages ahead into registers
+// and one into a double buffer in LDS, and each stage ends in one barrier.
+// The fp32 sums of a row run in K order whatever its chunk; only the
+// one-token stream sums in another order, and the stable placement gives
+// every row the same chunk on every call, so the output is bit-identical run
+// to run.
+//
+// Why this shape (Q4_K experts of 2048 x 768, 128 of them, 8 a token, both
+// GEMMs in one launch): the work is bound by the vector instructions that
+// dequantise, the clock falls under the load, and a batch of 512 tokens
+// leaves 32 rows an expert.  Eight wavefronts that dequantised 128 rows
+// into f16 LDS tiles for chunks of 128 rows spent most of their time at the
+// barrier behind the dequantisation and filled half a tile: 512 tokens took
+// 166 us, 1024 251 us, 37 79.6 us (whole calls); 64-row chunks, a fragment
+// dequantised where it is used and four small blocks a CU that cover each
+// other's waits: 143 us, 219 us, 71 us.  Wavefronts that held 128 rows each
+// (two blocks a CU, half the dequantisation for full chunks) measured 156 us
+// and 226 us: the batch rarely fills them.
 //
 // f16 rather than bf16 tiles: a Q4_K nibble q becomes the exact f16 1024 + q
 // (or 1024 + 16 q) with one v_and_or (its bits in the mantissa under 1024's
@@ -61,11 +73,10 @@ typedef _Float16 half2v __attribute__((ext_vector_type(2)));
 
 namespace {
 
-constexpr int MC = 128;       // sorted rows per chunk: 4 wavefronts x 32
-constexpr int KS = 128;       // K per stage: half a Q4_K super-block
-constexpr int LDK = KS;       // LDS row (f16 elements), units swizzled (bunit)
-constexpr int NB = 128;       // weight rows per block (gate/up: 64 gate + 64 up)
-constexpr int BN1 = 64;       // gate/up output columns per block
+constexpr int MC = 64;        // sorted rows per chunk: one or two token tiles of 32
+constexpr int KS = 64;        // K per stage: a sub-block pair of a Q4_K super-block
+constexpr int PT = 256;       // threads of a GEMM block: 4 wavefronts of 32 weight rows
+constexpr int BN1 = 64;       // gate/up output columns per block (16 a wavefront)
 constexpr int BN2 = 128;      // down output rows (= output columns of Y) per block
 
 size_t align256(size_t b) { return (b + 255) & ~(size_t)255; }
@@ -74,8 +85,7 @@ struct Ws {
     float *logits;
     uint32_t *ids;
     float *w;
-    int *offsets;   // [E+1]
-    int *chunks;    // [max_chunks][3] = (expert, first row, rows)
+    int *chunks;    // [max_chunks][3] = (expert, first sorted row, rows)
     int *n_chunks;  // [1]
     int *perm;      // [T*k] token of each sorted row
     int *pos;       // [T*k] sorted row of assignment t*k + s
@@ -95,7 +105,6 @@ Ws carve(void *base, int T, int k, int E, int Kd, int D) {
     w.logits = (float *)p; p += align256((size_t)T * E * 4);
     w.ids = (uint32_t *)p; p += align256(TK * 4);
     w.w = (float *)p; p += align256(TK * 4);
-    w.offsets = (int *)p; p += align256((size_t)(E + 1) * 4);
     w.chunks = (int *)p; p += align256((size_t)max_chunks((int)TK, E) * 12);
     w.n_chunks = (int *)p; p += 256;
     w.perm = (int *)p; p += align256(TK * 4);
@@ -108,255 +117,200 @@ Ws carve(void *base, int T, int k, int E, int Kd, int D) {
     return w;
 }
 
-// LDS weight tiles: a row's 128 K values are 16 units of 8 f16 (16 bytes);
-// unit u of row r is stored at unit bunit(r, u) = u ^ g(r) ^ 4 (u >> 3 & 1),
-// g(r) = r & 7 | (r >> 3 ^ r >> 1 & 1) << 3.  g takes 16 distinct values over
-// 16 consecutive rows, so the MFMA operand reads (consecutive lanes: rows
-// r.., one unit) fall in distinct 16-byte bank groups; the 4 (u >> 3 & 1)
-// separates a dequantising quad's units U and 8 + U of one row, so its
-// 16-byte writes (a quad per row, four rows per 16 lanes) are conflict-free
-// too, whether the LDS serves 8 lanes over 32 banks or 16 over 64.  A
-// bijection within each row (XOR with 4 leaves bit 3 alone).  Rows r and
-// r + 32 j share g.
-__host__ __device__ __forceinline__ int bunit(int r, int u) {
-    return u ^ ((r & 7) | (((r >> 3) ^ (r >> 1)) & 1) << 3) ^ (((u >> 3) & 1) << 2);
-}
+// LDS token tiles: a row's 64 K values are 8 units of 8 f16 (16 bytes); unit u
+// of row r is stored at unit u ^ aswz(r), so that the MFMA operand reads
+// (consecutive lanes: consecutive rows, one unit) of 16 rows fall in distinct
+// 16-byte bank groups (two rows to the 64 banks).
+__host__ __device__ __forceinline__ int aswz(int r) { return (r >> 1) & 7; }
 
 // The K order of every f16 operand: within each aligned group of 4 the
 // middle two elements are swapped (an involution).
 __host__ __device__ __forceinline__ int kperm(int c) { return (c & ~3) | ((c & 1) << 1) | ((c >> 1) & 1); }
 
-// 4 packed words of (1024 + q 2^j) pairs -> (scale q + neg_min) pairs
-// (scale already divided by 2^j), stored as 8 f16 at dst.
-__device__ __forceinline__ void q4_pairs_to_f16(const uint32_t (&v)[4], half2v sc, half2v nm, _Float16 *dst) {
+// The (1024 + q 2^j) pairs of a fragment -> (scale q + neg_min) pairs (scale
+// already divided by 2^j): 8 weights of the MFMA's B operand.
+__device__ __forceinline__ f16x8 q4_frag(uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3, half2v sc, half2v nm) {
     const half2v k1024 = {(_Float16)1024.0f, (_Float16)1024.0f};
+    const uint32_t v[4] = {v0, v1, v2, v3};
     uint32_t o[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const half2v q = __builtin_bit_cast(half2v, v[i]) - k1024;  // exact: q 2^j, q in 0..15
         o[i] = __builtin_bit_cast(uint32_t, q * sc + nm);
     }
-    *reinterpret_cast<uint4 *>(dst) = make_uint4(o[0], o[1], o[2], o[3]);
+    return __builtin_bit_cast(f16x8, make_uint4(o[0], o[1], o[2], o[3]));
 }
 
-// Q4_K 16-byte chunk cc (0..7) of a super-block with header hdr, dequantised
-// (quant/dequant.zig:157-187: (d*sc)*q - dmin*mn) to f16: elements 64p +
-// 16(cc&1) + [0, 8) at dst[0], + [8, 16) at dst[1], the same + 32 at dst[2],
-// dst[3] (p = cc / 2), each run in kperm order.  Quant byte j holds element j of the low run in its
-// low nibble and of the high run in its high nibble.  Under f16's exponent
-// of 1024 (0x6400) a nibble in mantissa bits 0-3 reads 1024 + q and one in
-// bits 4-7 reads 1024 + 16 q, both exact, so (w & 0x000f000f) | 0x64006400
-// is the low-run pair (e0, e2) of the word's bytes 0 and 2, (w & 0x00f000f0)
-// | 0x64006400 the high-run pair, and the same of w >> 8 gives (e1, e3):
-// one v_and_or per pair (the masks kept in registers so that the compiler
-// forms it), the high run's scale divided by 16.
-__device__ __forceinline__ void q4k_chunk_to_f16(uint4 hdr, uint4 q, int cc, _Float16 *const (&dst)[4]) {
-    const float d = f16_bits_to_f32(hdr.x), dmin = f16_bits_to_f32(hdr.x >> 16);
-    const int p = cc >> 1;
-    const int sh = (p & 1) * 16;
-    const uint32_t ys = hdr.y >> sh, zs = hdr.z >> sh, ws = hdr.w >> sh;
-    const uint32_t scp = opaque(p < 2 ? (ys & 0x3f3fu) : ((ws & 0x0f0fu) | ((ys >> 2) & 0x3030u)));
-    const uint32_t mnp = opaque(p < 2 ? (zs & 0x3f3fu) : (((ws >> 4) & 0x0f0fu) | ((zs >> 2) & 0x3030u)));
-    const _Float16 d1 = (_Float16)(d * (float)(scp & 0xffu)), m1 = (_Float16)(-(dmin * (float)(mnp & 0xffu)));
-    const _Float16 d2 = (_Float16)(d * (float)((scp >> 8) & 0xffu) * 0.0625f);
-    const _Float16 m2 = (_Float16)(-(dmin * (float)((mnp >> 8) & 0xffu)));
-    const uint32_t ml = opaque(0x000f000fu), mh = opaque(0x00f000f0u), ex = opaque(0x64006400u);
-    const uint32_t wv[4] = {q.x, q.y, q.z, q.w};
-    uint32_t lo[8], hi[8];
-#pragma unroll
-    for (int t = 0; t < 4; t++) {
-        const uint32_t w = wv[t], w8 = w >> 8;
-        lo[2 * t] = (w & ml) | ex;
-        lo[2 * t + 1] = (w8 & ml) | ex;
-        hi[2 * t] = (w & mh) | ex;
-        hi[2 * t + 1] = (w8 & mh) | ex;
-    }
-    const uint32_t lo0[4] = {lo[0], lo[1], lo[2], lo[3]}, lo1[4] = {lo[4], lo[5], lo[6], lo[7]};
-    const uint32_t hi0[4] = {hi[0], hi[1], hi[2], hi[3]}, hi1[4] = {hi[4], hi[5], hi[6], hi[7]};
-    q4_pairs_to_f16(lo0, half2v{d1, d1}, half2v{m1, m1}, dst[0]);
-    q4_pairs_to_f16(lo1, half2v{d1, d1}, half2v{m1, m1}, dst[1]);
-    q4_pairs_to_f16(hi0, half2v{d2, d2}, half2v{m2, m2}, dst[2]);
-    q4_pairs_to_f16(hi1, half2v{d2, d2}, half2v{m2, m2}, dst[3]);
-}
-
-// One thread's share of a K stage's weight tile: 2 units of (weight row r,
-// 16-byte chunk c): r = tid / 4 + 64 j, c = tid % 4.  The four threads of a
-// row (an aligned quad) each load one word of the row's 16-byte header and
-// share them over DPP, so a stage in flight holds 10 registers, not 16.
-struct StageRegs {
-    uint32_t h[2];
-    uint4 q[2];
+struct NoWait {
+    __device__ __forceinline__ void operator()() const {}
 };
 
-__device__ __forceinline__ void stage_load(StageRegs &R, const uint8_t *hdr, const uint8_t *qs, int nsb,
-                                           const size_t (&wrow)[2], int ks, int c) {
-    const int sb = ks >> 1, cc = (ks & 1) * 4 + c;
-#pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const size_t blk = wrow[j] * nsb + sb;
-        R.h[j] = *reinterpret_cast<const uint32_t *>(hdr + blk * 16 + 4 * c);
-        R.q[j] = ldg16(qs + blk * 128 + cc * 16);
-    }
-}
+// LDS of a GEMM block (40 KB: four blocks a CU): the token tiles' two stages
+// (after the GEMM the chunk's row scales), and per wavefront one super-block
+// of its 32 weight rows as loaded (128 bytes a row) and the headers of up to
+// 4 super-blocks (16 bytes each, 64 a row).
+struct __attribute__((aligned(16))) GemmLds {
+    _Float16 tok[2 * MC * KS];
+    uint4 quants[PT / 64][256], heads[PT / 64][128];
+};
 
-template <int CTRL>
-__device__ __forceinline__ uint32_t quad_word(uint32_t v) {
-    return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xf, 0xf, true);
-}
-
-// Stage ks's chunk cc = 4 (ks & 1) + c lands at local K 64 (c / 2) + 16 (c & 1)
-// (low nibbles) and +32 (high nibbles): units U, U + 1, U + 4, U + 5 with U
-// = 8 (c / 2) + 2 (c & 1), at doff[q] = 8 bunit(r0, unit) (rows r0 + 64 j
-// share r0's swizzle).
-__device__ __forceinline__ void stage_dequant(const StageRegs &R, _Float16 (*Bs)[LDK], int r0, int ks, int c,
-                                              const int (&doff)[4]) {
-    const int cc = (ks & 1) * 4 + c;
+// The grouped GEMM of one wavefront: its 32 weight rows against the chunk's
+// MT token tiles of 32, K = 256 nsb.  Every wavefront of the block works on
+// the same tokens and rows of its own.
+// Weights: the MFMA wants lane l to hold row l & 31, whose rows are a row
+// length apart in memory -- loaded that way each 16-byte load touches 32
+// cache lines and takes about 100 cycles of the CU's load path, more than the
+// MFMAs that use it.
+// So eight lanes load a row's 128 bytes, eight rows a load, and the words
+// cross to their lanes through a buffer in LDS that only this wavefront uses;
+// the LDS sees a wavefront's accesses in order, so a super-block is written
+// as soon as the one before has been read.  goff[j] is the byte offset of row
+// 8 j + (lane >> 3) in the quant plane (8 times that in the header plane).
+// Dequantised (quant/dequant.zig:157-187: (d*sc)*q - dmin*mn) straight into
+// the B fragments, the weights are never written again.  K is taken in the
+// order the nibbles come: the lane's 16 bytes of pair p are bytes 16 (lane >>
+// 5) of the pair's 32, and fragment (pair, low or high nibble, half j of the
+// 16) holds elements 64 p + 32 hi + 16 (lane >> 5) + 8 j + [0, 8), each
+// aligned 4 with its middle two swapped (kperm); the token tile is read in
+// the same order.  Under f16's exponent of 1024 (0x6400) a nibble in mantissa
+// bits 0-3 reads 1024 + q and one in bits 4-7 reads 1024 + 16 q, both exact:
+// one v_and_or a pair of weights (the masks kept in registers so that the
+// compiler forms it), the high nibbles' scale divided by 16.
+// Tokens: each thread loads 16 bytes of one row of every tile a stage (K =
+// 64) into registers, two stages ahead, and writes them to the LDS buffer
+// that the stage before has read; one barrier a stage.  aoff counts units of
+// 16 bytes (65536 rows of any length pass 4 GB).
+// All loads are unconditional (stages past the end clamped, their data left
+// unused), so that the waits count what is in flight.  wait() runs in every
+// thread once the first weights are requested and before the first token
+// load.
+template <int MT, typename Wait>
+__device__ __forceinline__ void gemm_tiles(floatx16 (&acc)[MT], GemmLds &L, const uint8_t *hdr, const uint8_t *qs,
+                                           uint32_t up, int nsb, const uint8_t *abase, const uint32_t (&aoff)[MT],
+                                           int wave, int tid, int lane, Wait wait) {
+    constexpr int TB = MT * 32 * KS;  // f16 per token buffer
+    constexpr bool kWaits = !__is_same(Wait, NoWait);
+    const int NS = 4 * nsb;
+    uint4 Q[4], A[2][MT];
+    const int lr = lane >> 3, lc = lane & 7;  // a load's row 8 j + lr, word lc
+    const int row = lane & 31, half = lane >> 5;
+    // rows 8 j + lr of the wavefront's weights: j = 2, 3 are `up` rows behind j = 0, 1
+    const uint32_t pitch = (uint32_t)nsb * 128u, goff = (uint32_t)lr * pitch + 16u * lc;
+    auto jrow = [&](int j) { return (j & 1) * 8u + (j >= 2 ? up : 0u); };
+    auto qld = [&](int sb) {
+        const uint8_t *p = qs + (size_t)min(sb, nsb - 1) * 128;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        _Float16 *row = Bs[r0 + 64 * j];
-        const uint4 h = make_uint4(quad_word<0x00>(R.h[j]), quad_word<0x55>(R.h[j]), quad_word<0xAA>(R.h[j]),
-                                   quad_word<0xFF>(R.h[j]));
-        _Float16 *const dst[4] = {row + doff[0], row + doff[1], row + doff[2], row + doff[3]};
-        q4k_chunk_to_f16(h, R.q[j], cc, dst);
+        for (int j = 0; j < 4; j++) Q[j] = ldg16(p + (size_t)jrow(j) * pitch + goff);
+    };
+    // word c of row r stands at byte 128 r + 16 (c ^ (r >> 1 & 7)) of the
+    // wavefront's quants: for row 8 j + lr that is 1024 j + 128 lr + 16 ((lc ^
+    // lr >> 1) ^ 4 (j & 1)), so that one address register serves all four
+    uint8_t *const wq = reinterpret_cast<uint8_t *>(L.quants[wave]);
+    const uint32_t qwr = 128u * lr + 16u * (lc ^ (lr >> 1)), qrd = 128u * row + 16u * (half ^ ((row >> 1) & 7));
+    auto qput = [&] {
+        const uint32_t b = opaque(qwr);
+#pragma unroll
+        for (int j = 0; j < 4; j++) *reinterpret_cast<uint4 *>(wq + ((b ^ (64u * (j & 1))) + 1024u * j)) = Q[j];
+    };
+    // headers of super-blocks sb + [0, 4), word c of row r at byte 64 r + 16
+    // (c ^ (r >> 2 & 3)): lane words 0-3 load rows 8 j + lr for j = 0, 1, the
+    // others for j = 2, 3
+    uint8_t *const wh = reinterpret_cast<uint8_t *>(L.heads[wave]);
+    const int hr = 16 * (lc >> 2) + lr, hc = lc & 3;
+    auto hld = [&](uint4 (&r)[2], int sb) {
+        const uint8_t *p =
+            hdr + (size_t)min(sb + hc, nsb - 1) * 16 + (size_t)((lc >> 2 ? up : 0u) + lr) * (uint32_t)(nsb * 16);
+        r[0] = ldg16(p);
+        r[1] = ldg16(p + nsb * 128);
+    };
+    auto hput = [&](const uint4 (&r)[2]) {
+        *reinterpret_cast<uint4 *>(wh + 64 * hr + 16 * (hc ^ ((hr >> 2) & 3))) = r[0];
+        *reinterpret_cast<uint4 *>(wh + 64 * (hr + 8) + 16 * (hc ^ (((hr + 8) >> 2) & 3))) = r[1];
+    };
+    const uint32_t hrd = 64u * row + 16u * ((row >> 2) & 3);
+    auto ald = [&](uint4 (&r)[MT], int st) {
+        const uint32_t k = (uint32_t)min(st, NS - 1) * (KS / 8);
+#pragma unroll
+        for (int t = 0; t < MT; t++) r[t] = ldg16(abase + ((uint64_t)(aoff[t] + k) << 4));
+    };
+    _Float16 *const aw = L.tok + (tid >> 3) * KS + 8 * ((tid & 7) ^ aswz(tid >> 3));
+    auto awr = [&](const uint4 (&r)[MT], int buf) {
+#pragma unroll
+        for (int t = 0; t < MT; t++) *reinterpret_cast<uint4 *>(aw + buf * TB + t * 32 * KS) = r[t];
+    };
+#pragma unroll
+    for (int t = 0; t < MT; t++) acc[t] = floatx16{};
+    uint4 h0[2];
+    hld(h0, 0);
+    qld(0);
+    if (!kWaits) {
+        ald(A[0], 0);
+        ald(A[1], 1);
     }
-}
-
-// The grouped GEMM of one block over the chunk's rows and the block's NB
-// weight rows (ct = 0..3 tiles of 32), K = 128 * NS.  Wavefront w takes
-// token tile t = w % (4 / S) and, of every stage's 8 K steps of 16, the
-// steps [kb, kb + 8 / S) with kb = (w / (4 / S)) * 8 / S: S = 1 gives each
-// of 4 tiles a wavefront of its own; S = 2 / 4 split the K steps of 2 / 1
-// tiles over 2 / 4 wavefronts, so a chunk with a single token tile still
-// keeps all four wavefronts' MFMA pipes busy.  arow points at this lane's A
-// row (row 32 t + lane % 32 of the chunk) plus its K half (lane / 32) * 8.
-// wait() runs (in every thread) once the first weight stages are requested
-// and before the first A load: the fused kernel's down blocks wait there
-// for their chunk's activations.
-template <int S, typename Wait>
-__device__ __forceinline__ void grouped_gemm(floatx16 (&acc)[4], _Float16 (*Bs)[NB][LDK], const uint8_t *hdr,
-                                             const uint8_t *qs, int nsb, const size_t (&wrow)[2], int NS,
-                                             const _Float16 *arow, bool wave_on, int kb, int tid, int lane,
-                                             Wait wait) {
-    constexpr int NK = 8 / S;
-    const int c = tid & 3, r0 = tid >> 2;
-    int doff[4], boff[NK];  // this thread's swizzled LDS units (f16 offsets in a row)
-    {
-        const int U = 8 * (c >> 1) + 2 * (c & 1);
-        doff[0] = 8 * bunit(r0, U);
-        doff[1] = 8 * bunit(r0, U + 1);
-        doff[2] = 8 * bunit(r0, U + 4);
-        doff[3] = 8 * bunit(r0, U + 5);
-#pragma unroll
-        for (int i = 0; i < NK; i++) boff[i] = 8 * bunit(lane & 31, 2 * (kb + i) + (lane >> 5));
+    hput(h0);
+    qput();
+    qld(1);
+    if (kWaits) {
+        wait();
+        ald(A[0], 0);
+        ald(A[1], 1);
     }
-    StageRegs R[3];
-    f16x8 a[2][NK];
-#pragma unroll
-    for (int i = 0; i < 4; i++) acc[i] = floatx16{};
-    // Every wavefront issues the same loads on every path (stage indices
-    // past the end are clamped and their data left unused; a wavefront
-    // without a token tile loads a valid row it does not use): the memory
-    // counter waits the compiler derives then cover only the data a step
-    // needs, not the prefetches behind it.  Three stages' weights are in
-    // flight ahead of the one being dequantised.
-    stage_load(R[0], hdr, qs, nsb, wrow, 0, c);
-    stage_load(R[1], hdr, qs, nsb, wrow, 1, c);  // NS = 2 * super-blocks >= 2
-    stage_load(R[2], hdr, qs, nsb, wrow, min(2, NS - 1), c);
-    wait();
-#pragma unroll
-    for (int i = 0; i < NK; i++) a[0][i] = *reinterpret_cast<const f16x8 *>(arow + (kb + i) * 16);
-    stage_dequant(R[0], Bs[0], r0, 0, c, doff);
-    stage_load(R[0], hdr, qs, nsb, wrow, min(3, NS - 1), c);
+    awr(A[0], 0);
+    ald(A[0], 2);
+    // fragment (pp, hi, j) of row lane & 31 is unit K + 2 (lane >> 5), K = 8
+    // pp + 4 hi + j, at byte 256 row + 16 ((K ^ 2 (lane >> 5)) ^ aswz(row))
+    const uint32_t trd = 128u * row + 16u * (aswz(row) ^ (2 * half));
+    const uint8_t *const tok = reinterpret_cast<const uint8_t *>(L.tok);
+    uint32_t ml = 0x000f000fu, mh = 0x00f000f0u;
+    asm volatile("" : "+s"(ml), "+s"(mh));
+    const uint32_t ex = opaque(0x64006400u);
     __syncthreads();
-    // Six stages per trip, so that the A buffers (stage parity) and the
-    // weight register sets (stage mod 3) have fixed names: entering stage
-    // st, Bs[st & 1] holds it and R[(st + 1) % 3], R[(st + 2) % 3],
-    // R[st % 3] hold stages st + 1, st + 2, st + 3.
-    for (int ks = 0; ks < NS; ks += 6) {
+    for (int sb = 0; sb < nsb; sb++) {
+        if ((sb & 3) == 0 && sb) {
+            uint4 r[2];
+            hld(r, sb);
+            hput(r);
+        }
+        const uint4 h = *reinterpret_cast<const uint4 *>(wh + (hrd ^ (16u * (sb & 3))));
+        const float d = f16_bits_to_f32(h.x), dmin = f16_bits_to_f32(h.x >> 16);
 #pragma unroll
-        for (int u = 0; u < 6; u++) {
-            const int st = ks + u;
-            if (st >= NS) break;  // (uniform over the block)
-            StageRegs &Rn = R[(u + 1) % 3];  // stage st + 1
-            f16x8(&acur)[NK] = a[u & 1];
-            f16x8(&anext)[NK] = a[(u + 1) & 1];
-            const size_t sa = (size_t)min(st + 1, NS - 1) * KS;
-#pragma unroll
-            for (int i = 0; i < NK; i++) anext[i] = *reinterpret_cast<const f16x8 *>(arow + sa + (kb + i) * 16);
-            if (wave_on) {
-                _Float16(*B)[LDK] = Bs[st & 1];
-#pragma unroll
-                for (int i = 0; i < NK; i++)
-#pragma unroll
-                    for (int ct = 0; ct < 4; ct++) {
-                        const f16x8 b = *reinterpret_cast<const f16x8 *>(&B[32 * ct + (lane & 31)][boff[i]]);
-                        acc[ct] = __builtin_amdgcn_mfma_f32_32x32x16_f16(acur[i], b, acc[ct], 0, 0, 0);
-                    }
+        for (int p = 0; p < 4; p++) {
+            const int st = 4 * sb + p;
+            const uint4 q = *reinterpret_cast<const uint4 *>(wq + (opaque(qrd) ^ (32u * p)));
+            if (p == 3) {  // the super-block has been read: the next one in its place
+                qput();
+                qld(sb + 2);
             }
-            if (st + 1 < NS) stage_dequant(Rn, Bs[(st + 1) & 1], r0, st + 1, c, doff);
-            stage_load(Rn, hdr, qs, nsb, wrow, min(st + 4, NS - 1), c);
+            awr(A[(p + 1) & 1], (p + 1) & 1);  // (past the end: a buffer nobody reads any more)
+            ald(A[(p + 1) & 1], st + 3);
+            const uint32_t tb = opaque(trd);
+            // get_scale_min_k4 of sub-blocks 2 p, 2 p + 1
+            const uint32_t ys = h.y >> (16 * (p & 1)), zs = h.z >> (16 * (p & 1)), ws = h.w >> (16 * (p & 1));
+            const uint32_t scp = opaque(p < 2 ? (ys & 0x3f3fu) : ((ws & 0x0f0fu) | ((ys >> 2) & 0x3030u)));
+            const uint32_t mnp = opaque(p < 2 ? (zs & 0x3f3fu) : (((ws >> 4) & 0x0f0fu) | ((zs >> 2) & 0x3030u)));
+            const _Float16 d1 = (_Float16)(d * (float)(scp & 0xffu));
+            const _Float16 m1 = (_Float16)(-(dmin * (float)(mnp & 0xffu)));
+            const _Float16 d2 = (_Float16)(d * (float)((scp >> 8) & 0xffu) * 0.0625f);
+            const _Float16 m2 = (_Float16)(-(dmin * (float)((mnp >> 8) & 0xffu)));
+            const uint32_t qw[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+            for (int f = 0; f < 4; f++) {  // 2 hi + j
+                f16x8 a[MT];
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    a[t] = *reinterpret_cast<const f16x8 *>(tok + (tb ^ (16u * (4 * (f >> 1) + (f & 1)))) +
+                                                            2 * ((p & 1) * TB + t * 32 * KS));
+                const uint32_t w0 = qw[2 * (f & 1)], w1 = qw[2 * (f & 1) + 1], m = f < 2 ? ml : mh;
+                const half2v sc = f < 2 ? half2v{d1, d1} : half2v{d2, d2};
+                const half2v nm = f < 2 ? half2v{m1, m1} : half2v{m2, m2};
+                const f16x8 b =
+                    q4_frag((w0 & m) | ex, ((w0 >> 8) & m) | ex, (w1 & m) | ex, ((w1 >> 8) & m) | ex, sc, nm);
+#pragma unroll
+                for (int t = 0; t < MT; t++)
+                    acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a[t], b, acc[t], 0, 0, 0);
+            }
             __syncthreads();
         }
-    }
-}
-
-// Runs the block's GEMM with K split S and hands every finished C element to
-// epi(tile t, element i, values of the 4 column tiles): for S > 1 the S
-// partial sums of a tile meet in LDS (the weight buffers, free after the
-// last stage) and are added in wavefront order, so results do not depend
-// on timing.  acc element i of a 32x32 tile is C[(i / 4) * 8 + (lane / 32) *
-// 4 + i % 4][lane % 32].
-// pre(t, i) gives a value epi receives with element i (the gate/up
-// kernel's row scale): all of a wavefront's pre loads are issued before its
-// first epi, so that their round trips overlap instead of queueing behind
-// each element's stores.
-template <int S, typename Row, typename Pre, typename Epi, typename Wait>
-__device__ __forceinline__ void run_block(_Float16 (*Bs)[NB][LDK], const uint8_t *hdr, const uint8_t *qs, int nsb,
-                                          const size_t (&wrow)[2], int NS, int mc, Row row_ptr, Pre pre, Epi epi,
-                                          Wait wait, int tid, int wave, int lane) {
-    constexpr int NT = 4 / S;  // token tiles handled side by side
-    const int t = wave % NT, q = wave / NT;
-    const int mrow = 32 * t + (lane & 31);
-    const bool wave_on = 32 * t < mc;
-    const _Float16 *arow = row_ptr(mrow < mc ? mrow : 0) + (lane >> 5) * 8;
-    floatx16 acc[4];
-    grouped_gemm<S>(acc, Bs, hdr, qs, nsb, wrow, NS, arow, wave_on, q * (8 / S), tid, lane, wait);
-    constexpr int NI = 16 / S;  // elements this wavefront hands over
-    const int i0 = S == 1 ? 0 : q * NI;
-    float pv[NI];
-    if (S == 1) {
-        if (wave_on) {
-#pragma unroll
-            for (int ii = 0; ii < NI; ii++) pv[ii] = pre(t, ii);
-#pragma unroll
-            for (int i = 0; i < 16; i++) {
-                const float v[4] = {acc[0][i], acc[1][i], acc[2][i], acc[3][i]};
-                epi(t, i, v, pv[i]);
-            }
-        }
-        return;
-    }
-    float *red = reinterpret_cast<float *>(&Bs[0][0][0]);  // [4 waves][4 ct][16 i][64 lanes]
-#pragma unroll
-    for (int ct = 0; ct < 4; ct++)
-#pragma unroll
-        for (int i = 0; i < 16; i++) red[((wave * 4 + ct) * 16 + i) * 64 + lane] = acc[ct][i];
-    __syncthreads();
-    if (!wave_on) return;
-#pragma unroll
-    for (int ii = 0; ii < NI; ii++) pv[ii] = pre(t, i0 + ii);
-#pragma unroll
-    for (int ii = 0; ii < NI; ii++) {
-        const int i = i0 + ii;
-        float v[4];
-#pragma unroll
-        for (int ct = 0; ct < 4; ct++) {
-            float sum = 0.0f;
-#pragma unroll
-            for (int qq = 0; qq < S; qq++) sum += red[(((t + NT * qq) * 4 + ct) * 16 + i) * 64 + lane];
-            v[ct] = sum;
-        }
-        epi(t, i, v, pv[ii]);
     }
 }
 
@@ -404,8 +358,8 @@ __device__ __forceinline__ int rank_in(uint64_t m) {
 // and kept with their ranks for the placement; longer batches read them
 // again.
 __global__ void __launch_bounds__(1024) k_prefill_dispatch(const uint32_t *__restrict__ ids, int TK, int k, int E,
-                                                           int *__restrict__ offsets, int *__restrict__ chunks,
-                                                           int *__restrict__ n_chunks, int *__restrict__ perm,
+                                                           int *__restrict__ chunks, int *__restrict__ n_chunks,
+                                                           int *__restrict__ perm,
                                                            int *__restrict__ pos, int *__restrict__ done, int maxc) {
     constexpr int kIdsPer = 8, kTab = 16384;
     __shared__ int cnt[1024], cur[1024], psum[1024];
@@ -475,59 +429,51 @@ __global__ void __launch_bounds__(1024) k_prefill_dispatch(const uint32_t *__res
     // first and the short ones fill in behind them.
     if (wave == 0) {
         const int CH = (E + 63) >> 6;
-        int t0 = 0, t1 = 0, t12 = 0, t34 = 0;  // rows, full chunks, partial chunks of 1 | 2 << 16, 3 | 4 << 16 tiles
+        int t0 = 0, t1 = 0, t12 = 0;  // rows, full chunks, partial chunks of 1 | 2 << 16 tiles
         for (int q = 0; q < CH; q++) {
             const int e = CH * lane + q;
             const int n = e < E ? cnt[e] : 0, rem = n % MC, cls = rem ? (rem + 31) / 32 : 0;
             t0 += n;
             t1 += n / MC;
             t12 += (cls == 1 ? 1 : 0) + (cls == 2 ? 0x10000 : 0);
-            t34 += (cls == 3 ? 1 : 0) + (cls == 4 ? 0x10000 : 0);
         }
-        int i0 = t0, i1 = t1, i12 = t12, i34 = t34;  // inclusive scans over the lanes
+        int i0 = t0, i1 = t1, i12 = t12;  // inclusive scans over the lanes
 #pragma unroll
         for (int d = 1; d < 64; d <<= 1) {
             const int a0 = __shfl_up(i0, d, 64), a1 = __shfl_up(i1, d, 64);
-            const int a12 = __shfl_up(i12, d, 64), a34 = __shfl_up(i34, d, 64);
+            const int a12 = __shfl_up(i12, d, 64);
             if (lane >= d) {
                 i0 += a0;
                 i1 += a1;
                 i12 += a12;
-                i34 += a34;
             }
         }
-        const int T1 = __shfl(i1, 63, 64), T12 = __shfl(i12, 63, 64), T34 = __shfl(i34, 63, 64);
-        const int tot_full = T1, tot_p4 = T34 >> 16, tot_p3 = T34 & 0xffff, tot_p2 = T12 >> 16, tot_p1 = T12 & 0xffff;
+        const int tot_full = __shfl(i1, 63, 64), T12 = __shfl(i12, 63, 64);
+        const int tot_p2 = T12 >> 16, tot_p1 = T12 & 0xffff;
         // first chunk index of each partial class, then this lane's running positions
         int off = i0 - t0, fc = i1 - t1;
-        int pc[4] = {tot_full + tot_p4 + tot_p3 + tot_p2 + ((i12 - t12) & 0xffff),
-                     tot_full + tot_p4 + tot_p3 + ((i12 - t12) >> 16), tot_full + tot_p4 + ((i34 - t34) & 0xffff),
-                     tot_full + ((i34 - t34) >> 16)};
+        int pc[2] = {tot_full + tot_p2 + ((i12 - t12) & 0xffff), tot_full + ((i12 - t12) >> 16)};
         for (int q = 0; q < CH; q++) {
             const int e = CH * lane + q;
             if (e >= E) break;
             const int n = cnt[e], full = n / MC, rem = n % MC, cls = rem ? (rem + 31) / 32 : 0;
-            offsets[e] = off;
             cur[e] = off;
             for (int j = 0; j < full; j++) {
                 int *ch = chunks + 3 * (fc + j);
                 ch[0] = e;
-                ch[1] = j * MC;
+                ch[1] = off + j * MC;
                 ch[2] = MC;
             }
             fc += full;
             if (cls) {
                 int *ch = chunks + 3 * pc[cls - 1];
                 ch[0] = e;
-                ch[1] = full * MC;
+                ch[1] = off + full * MC;
                 ch[2] = rem;
                 pc[cls - 1]++;
             }
             off += n;
-            if (e == E - 1) {
-                offsets[E] = off;
-                *n_chunks = tot_full + tot_p4 + tot_p3 + tot_p2 + tot_p1;
-            }
+            if (e == E - 1) *n_chunks = tot_full + tot_p2 + tot_p1;
         }
     }
     __syncthreads();
@@ -648,7 +594,7 @@ struct PfArgs {
     const _Float16 *Xh;
     const float *rs;
     int D;
-    const int *chunks, *n_chunks, *offsets, *perm;
+    const int *chunks, *n_chunks, *perm;
     _Float16 *H;
     int Kd;
     const uint8_t *dn_hdr, *dn_qs;  // down planes: [E][D] rows of dn_nsb super-blocks
@@ -659,10 +605,6 @@ struct PfArgs {
     int CG;     // fused kernel: chunk slots per XCD group
     const float *X;  // the fp32 input rows (one-token chunks)
     int tiny;        // one-token chunks take the decode-style stream (gate/up rows <= 8, down rows <= 4 super-blocks)
-};
-
-struct NoWait {
-    __device__ __forceinline__ void operator()() const {}
 };
 
 // ---------------------------------------------------------------- chunks of one token
@@ -709,7 +651,7 @@ __device__ __forceinline__ float window_dot(const WinW &w, int p, const Limbs &x
 // position order.
 template <int ACT, int NT>
 __device__ __forceinline__ uint32_t gate_up_tiny(const PfArgs &a, float *red, const int *prow, int e, int row0,
-                                                 int n0, int wave, int lane) {
+                                                 int col0, int wave, int lane) {
     const int F = a.F, nsb = a.gu_nsb, Kd = a.Kd;
     const int pos = lane & 31, sb = min(pos >> 2, nsb - 1), p = pos & 3;
     const bool on = (pos >> 2) < nsb;
@@ -733,7 +675,7 @@ __device__ __forceinline__ uint32_t gate_up_tiny(const PfArgs &a, float *red, co
         xl[t].xs_hi = xs[2] + xs[3];
     }
     auto blk_of = [&](int c) {
-        const int col = n0 + 16 * wave + c;
+        const int col = col0 + c;
         return ((size_t)e * 2 * F + (half ? F + col : col)) * nsb + sb;
     };
     WinW w[16];
@@ -763,7 +705,7 @@ __device__ __forceinline__ uint32_t gate_up_tiny(const PfArgs &a, float *red, co
         const float h = prefill_act<ACT>(v) * up * ri * ri;
         const bool big = fabsf(h) > 65504.0f && fabsf(h) <= 3.4e38f;
         sat = big ? 1u : 0u;
-        a.H[(size_t)(row0 + t) * Kd + kperm(n0 + 16 * wave + c)] = (_Float16)(big ? copysignf(65504.0f, h) : h);
+        a.H[(size_t)(row0 + t) * Kd + kperm(col0 + c)] = (_Float16)(big ? copysignf(65504.0f, h) : h);
     }
     return sat;
 }
@@ -774,13 +716,13 @@ __device__ __forceinline__ uint32_t gate_up_tiny(const PfArgs &a, float *red, co
 // c < 8.  The activations are the H rows (f16, K in kperm order).  Lane
 // c + 8 rr + 32 t then sums the 16 positions of (pass c, row rr, token t).
 template <int NT, typename Wait>
-__device__ __forceinline__ void down_tiny(const PfArgs &a, float *red, int e, int row0, int n0, Wait wait, int wave,
+__device__ __forceinline__ void down_tiny(const PfArgs &a, float *red, int e, int row0, int nrow, Wait wait, int wave,
                                           int lane) {
     const int nsb = a.dn_nsb, D = a.D, Kd = a.Kd;
     const int pos = lane & 15, sb = min(pos >> 2, nsb - 1), p = pos & 3;
     const bool on = (pos >> 2) < nsb;
     const int rr = lane >> 4;
-    auto blk_of = [&](int c) { return ((size_t)e * D + n0 + 32 * wave + 4 * c + rr) * nsb + sb; };
+    auto blk_of = [&](int c) { return ((size_t)e * D + nrow + 4 * c + rr) * nsb + sb; };
     WinW w[8];
 #pragma unroll
     for (int c = 0; c < 2; c++) w[c] = load_window(a.dn_hdr, a.dn_qs, blk_of(c), p);
@@ -825,114 +767,156 @@ __device__ __forceinline__ void down_tiny(const PfArgs &a, float *red, int e, in
         float v = 0.0f;
 #pragma unroll
         for (int q = 0; q < 16; q++) v += src[q];
-        a.Y[(size_t)(row0 + t) * D + n0 + 32 * wave + 4 * c + r4] = v;
+        a.Y[(size_t)(row0 + t) * D + nrow + 4 * c + r4] = v;
     }
 }
 
-// Block: chunk (expert e, sorted rows base + m0 + [0, mc)) x output columns
-// [n0, n0 + 64).  Weight rows 0..63 are gate rows n0.., 64..127 the up rows;
-// wavefront w computes token tile w against all 128 (ct 0,1 = gate, 2,3 =
-// up), so h = act(gate) * up is formed in registers.  ACT: the activation
-// (0 SiLU, 1 GELU-tanh).  False when the chunk does not exist.
-template <int ACT>
-__device__ __forceinline__ bool gate_up_body(const PfArgs &a, int bx, int by, _Float16 (*Bs)[NB][LDK]) {
-    if (by >= *a.n_chunks) return false;
-    const int e = a.chunks[3 * by], m0 = a.chunks[3 * by + 1], mc = a.chunks[3 * by + 2];
-    const int base = a.offsets[e];
-    const int n0 = bx * BN1, F = a.F, D = a.D, Kd = a.Kd;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    size_t wrow[2];
+// acc element i of a 32 x 32 tile is C[tile_row(i, lane)][lane & 31].
+__device__ __forceinline__ int tile_row(int i, int lane) { return (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3); }
+
+// The tiles of a gate/up block: wavefront w has gate columns n0 + 16 w + [0,
+// 16) in its rows 0-15 and the matching up columns in rows 16-31.  The halves
+// trade values (element i's up against element i + 1's gate), so that lanes
+// 0-15 of a 32-lane half finish element i and lanes 16-31 element i + 1.
+// With r the token's row scale, gate = r g and up = r u, and H = act(gate) *
+// up / r^2 = act(r g) * (u / r) (exact scalings), stored in kperm order (the
+// down GEMM's K); a finite value past f16's range saturates at +-65504 and is
+// counted (inf and NaN pass through).
+template <int ACT, int MT>
+__device__ __forceinline__ uint32_t gate_up_tiles(const PfArgs &a, GemmLds &L, const int *prow, size_t wrow0, int row0,
+                                                  int mc, int col, int wave, int tid, int lane) {
+    floatx16 acc[MT];
+    uint32_t aoff[MT];
+    const float rt = a.rs[prow[min(tid, mc - 1)]];  // (rows past the chunk: its last row's)
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const int r = (tid >> 2) + 64 * j;
-        wrow[j] = (size_t)e * 2 * F + (r < BN1 ? n0 + r : F + n0 + (r - BN1));
+    for (int t = 0; t < MT; t++) {
+        const int m = 32 * t + (tid >> 3);
+        aoff[t] = (uint32_t)prow[m < mc ? m : 0] * (uint32_t)(a.D / 8) + (tid & 7);
     }
-    const int *prow = a.perm + base + m0;
-    const _Float16 *Xh = a.Xh;
-    const float *rs = a.rs;
-    _Float16 *H = a.H;
-    auto row_ptr = [&](int m) { return Xh + (size_t)prow[m] * D; };
-    // ct 0, 1 = gate columns n0 + [0, 64), ct 2, 3 = the matching up columns;
-    // with r the row's scale, gate = r v[0] and up = r v[2], and H = act(gate)
-    // * up / r^2 = act(r v[0]) * (v[2] / r) (exact scalings) is stored in
-    // kperm order (the down GEMM's K); a finite value past f16's range
-    // saturates at +-65504 and is counted (inf and NaN pass through)
+    gemm_tiles<MT>(acc, L, a.gu_hdr + wrow0 * a.gu_nsb * 16, a.gu_qs + wrow0 * a.gu_nsb * 128, (uint32_t)a.F,
+                   a.gu_nsb, reinterpret_cast<const uint8_t *>(a.Xh), aoff, wave, tid, lane, NoWait{});
+    // row scales r and 1 / r (r = 2^k exactly: frexp gives k + 1, so 1 / r = 2^(1 - (k + 1)))
+    float2 *const rs = reinterpret_cast<float2 *>(L.tok);  // (free behind the GEMM's last barrier)
+    if (tid < MC) rs[tid] = make_float2(rt, __builtin_amdgcn_ldexpf(1.0f, 1 - __builtin_amdgcn_frexp_expf(rt)));
+    __syncthreads();
+    // The block's H tile, 64 columns (128 bytes) a row, goes out through LDS in
+    // 16-byte stores.
     uint32_t sat = 0;
-    auto sat16 = [&](float h) {  // (no branch: a select and a count)
-        const bool big = fabsf(h) > 65504.0f && fabsf(h) <= 3.4e38f;
-        sat += big ? 1u : 0u;
-        return (_Float16)(big ? copysignf(65504.0f, h) : h);
-    };
-    auto pre = [&](int t, int i) {  // the row's scale (rows past the chunk: row 0's)
-        const int m = 32 * t + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-        return rs[prow[m < mc ? m : 0]];
-    };
-    auto epi = [&](int t, int i, const float (&v)[4], float r) {
-        const int m = 32 * t + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-        if (m < mc) {
-            // r = 2^k exactly: frexp gives k + 1, so 1 / r = 2^(1 - (k + 1))
-            const float ri = __builtin_amdgcn_ldexpf(1.0f, 1 - __builtin_amdgcn_frexp_expf(r));
-            _Float16 *hrow = H + (size_t)(base + m0 + m) * Kd;
-            const int c0 = n0 + (lane & 31);
-            hrow[kperm(c0)] = sat16(prefill_act<ACT>(v[0] * r) * (v[2] * ri));
-            hrow[kperm(c0 + 32)] = sat16(prefill_act<ACT>(v[1] * r) * (v[3] * ri));
+    const int up1 = (lane >> 4) & 1;
+    _Float16 *const ht = reinterpret_cast<_Float16 *>(L.tok) + 4 * MC + kperm(16 * wave + (lane & 15));
+    float top = 0.0f;
+    auto tile = [&](auto put) {
+#pragma unroll
+        for (int t = 0; t < MT; t++) {
+#pragma unroll
+            for (int i = 0; i < 16; i += 2) {
+                const float other = xor16(up1 ? acc[t][i] : acc[t][i + 1]);
+                const float g = up1 ? other : acc[t][i], u = up1 ? acc[t][i + 1] : other;
+                const int m = 32 * t + tile_row(i, lane) + up1;
+                const float2 r = rs[m];
+                put(m, prefill_act<ACT>(g * r.x) * (u * r.y));
+            }
         }
     };
-    const int nt = (mc + 31) / 32, NS = 2 * a.gu_nsb;
-    float *red = reinterpret_cast<float *>(&Bs[0][0][0]);
-    if (a.tiny && mc == 1)
-        sat = gate_up_tiny<ACT, 1>(a, red, prow, e, base + m0, n0, wave, lane);
-    else if (nt == 1)
-        run_block<4>(Bs, a.gu_hdr, a.gu_qs, a.gu_nsb, wrow, NS, mc, row_ptr, pre, epi, NoWait{}, tid, wave, lane);
-    else if (nt == 2)
-        run_block<2>(Bs, a.gu_hdr, a.gu_qs, a.gu_nsb, wrow, NS, mc, row_ptr, pre, epi, NoWait{}, tid, wave, lane);
-    else
-        run_block<1>(Bs, a.gu_hdr, a.gu_qs, a.gu_nsb, wrow, NS, mc, row_ptr, pre, epi, NoWait{}, tid, wave, lane);
+    tile([&](int m, float h) {
+        top = fmaxf(top, fabsf(h));
+        ht[BN1 * m] = (_Float16)h;
+    });
+    if (top > 65504.0f)  // (rare: rows in range and finite values saturate and count, inf and NaN stay)
+        tile([&](int m, float h) {
+            const bool big = fabsf(h) > 65504.0f && fabsf(h) <= 3.4e38f;
+            sat += big && m < mc ? 1u : 0u;
+            ht[BN1 * m] = (_Float16)(big ? copysignf(65504.0f, h) : h);
+        });
+    __syncthreads();
+    const int un = tid & 7;
+    _Float16 *const hout = a.H + (size_t)row0 * a.Kd + (col - 16 * wave) + 8 * un;
+#pragma unroll
+    for (int t = 0; t < MT; t++) {
+        const int m = 32 * t + (tid >> 3);
+        if (m < mc)
+            *reinterpret_cast<uint4 *>(hout + (size_t)m * (uint32_t)a.Kd) =
+                *reinterpret_cast<const uint4 *>(L.tok + 4 * MC + BN1 * m + 8 * un);
+    }
+    return sat;
+}
+
+// Block: chunk (expert e, sorted rows row0 + [0, mc)) x output columns n0 +
+// [0, 64).  ACT: the activation (0 SiLU, 1 GELU-tanh).  False when the
+// chunk does not exist.
+template <int ACT>
+__device__ __forceinline__ bool gate_up_body(const PfArgs &a, int bx, int by, GemmLds &L) {
+    if (by >= *a.n_chunks) return false;
+    const int e = __builtin_amdgcn_readfirstlane(a.chunks[3 * by]);
+    const int mc = __builtin_amdgcn_readfirstlane(a.chunks[3 * by + 2]);
+    const int row0 = __builtin_amdgcn_readfirstlane(a.chunks[3 * by + 1]);
+    const int n0 = bx * BN1, F = a.F, Kd = a.Kd;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int col = n0 + 16 * wave;  // this wavefront's 16 columns (F % 64 == 0)
+    const int *prow = a.perm + row0;
+    uint32_t sat = 0;
+    if (a.tiny && mc == 1) {
+        sat = gate_up_tiny<ACT, 1>(a, reinterpret_cast<float *>(L.tok), prow, e, row0, col, wave, lane);
+    } else {
+        // rows 8 j + (lane >> 3) of the wavefront: gate columns for j < 2, up columns for the others
+        const size_t wrow0 = (size_t)e * 2 * F + col;
+        sat = mc <= 32 ? gate_up_tiles<ACT, 1>(a, L, prow, wrow0, row0, mc, col, wave, tid, lane)
+                       : gate_up_tiles<ACT, 2>(a, L, prow, wrow0, row0, mc, col, wave, tid, lane);
+    }
     if (sat) {  // (rare): the count and the error bit, reported at the next synchronising call
         __hip_atomic_fetch_add(a.err + kErrPrefillSat, sat, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         report_timeout(a.err, kErrCodePrefillSat);
     }
     if (bx == 0 && Kd > F)  // zero K padding of the down product
-        for (int i = tid; i < mc * (Kd - F); i += 256) {
-            const int m = i / (Kd - F), col = F + i % (Kd - F);
-            H[(size_t)(base + m0 + m) * Kd + col] = (_Float16)0.f;  // (kperm keeps [F, Kd): F % 4 == 0)
+        for (int i = tid; i < mc * (Kd - F); i += PT) {
+            const int m = i / (Kd - F), c = F + i % (Kd - F);
+            a.H[(size_t)(row0 + m) * Kd + c] = (_Float16)0.f;  // (kperm keeps [F, Kd): F % 4 == 0)
         }
     return true;
 }
 
-// Block: chunk x output rows [n0, n0 + 128) of the expert's down matrix
-// (= columns of Y); wavefront w computes token tile w, A = H rows (f16).
-template <typename Wait>
-__device__ __forceinline__ void down_body(const PfArgs &a, int bx, int by, _Float16 (*Bs)[NB][LDK], Wait wait) {
-    const int e = a.chunks[3 * by], m0 = a.chunks[3 * by + 1], mc = a.chunks[3 * by + 2];
-    const int base = a.offsets[e];
-    const int n0 = bx * BN2, D = a.D, Kd = a.Kd;
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    size_t wrow[2];
+template <int MT, typename Wait>
+__device__ __forceinline__ void down_tiles(const PfArgs &a, GemmLds &L, size_t wrow0, int row0, int mc, int n, Wait wait,
+                                           int wave, int tid, int lane) {
+    floatx16 acc[MT];
+    uint32_t aoff[MT];
 #pragma unroll
-    for (int j = 0; j < 2; j++) wrow[j] = (size_t)e * D + n0 + (tid >> 2) + 64 * j;
-    const _Float16 *hbase = a.H + (size_t)(base + m0) * Kd;
-    float *Y = a.Y;
-    auto row_ptr = [&](int m) { return hbase + (size_t)m * Kd; };
-    auto pre = [](int, int) { return 0.0f; };
-    auto epi = [&](int t, int i, const float (&v)[4], float) {
-        const int m = 32 * t + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-        if (m < mc) {
-            float *yrow = Y + (size_t)(base + m0 + m) * D + n0 + (lane & 31);
+    for (int t = 0; t < MT; t++) {
+        const int m = 32 * t + (tid >> 3);
+        aoff[t] = (uint32_t)(m < mc ? m : 0) * (uint32_t)(a.Kd / 8) + (tid & 7);
+    }
+    gemm_tiles<MT>(acc, L, a.dn_hdr + wrow0 * a.dn_nsb * 16, a.dn_qs + wrow0 * a.dn_nsb * 128, 16u, a.dn_nsb,
+                   reinterpret_cast<const uint8_t *>(a.H + (size_t)row0 * a.Kd), aoff, wave, tid, lane, wait);
+    float *ycol = a.Y + (size_t)row0 * a.D + n + (lane & 31);
 #pragma unroll
-            for (int ct = 0; ct < 4; ct++) yrow[32 * ct] = v[ct];
+    for (int t = 0; t < MT; t++) {
+        const bool full = 32 * t + 32 <= mc;  // (uniform: no branch per element)
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const int m = 32 * t + tile_row(i, lane);
+            if (full || m < mc) ycol[(size_t)m * (uint32_t)a.D] = acc[t][i];
         }
-    };
-    const int nt = (mc + 31) / 32, NS = 2 * a.dn_nsb;
-    float *red = reinterpret_cast<float *>(&Bs[0][0][0]);
-    if (a.tiny && mc == 1)
-        down_tiny<1>(a, red, e, base + m0, n0, wait, wave, lane);
-    else if (nt == 1)
-        run_block<4>(Bs, a.dn_hdr, a.dn_qs, a.dn_nsb, wrow, NS, mc, row_ptr, pre, epi, wait, tid, wave, lane);
-    else if (nt == 2)
-        run_block<2>(Bs, a.dn_hdr, a.dn_qs, a.dn_nsb, wrow, NS, mc, row_ptr, pre, epi, wait, tid, wave, lane);
+    }
+}
+
+// Block: chunk x output rows n0 + [0, 128) of the expert's down matrix (=
+// columns of Y), 32 a wavefront; the token operand is the H rows (f16).
+template <typename Wait>
+__device__ __forceinline__ void down_body(const PfArgs &a, int bx, int by, GemmLds &L, Wait wait) {
+    const int e = __builtin_amdgcn_readfirstlane(a.chunks[3 * by]);
+    const int mc = __builtin_amdgcn_readfirstlane(a.chunks[3 * by + 2]);
+    const int row0 = __builtin_amdgcn_readfirstlane(a.chunks[3 * by + 1]);
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int n = bx * BN2 + 32 * wave;  // (D % 128 == 0)
+    if (a.tiny && mc == 1) {
+        down_tiny<1>(a, reinterpret_cast<float *>(L.tok), e, row0, n, wait, wave, lane);
+        return;
+    }
+    const size_t wrow0 = (size_t)e * a.D + n;
+    if (mc <= 32)
+        down_tiles<1>(a, L, wrow0, row0, mc, n, wait, wave, tid, lane);
     else
-        run_block<1>(Bs, a.dn_hdr, a.dn_qs, a.dn_nsb, wrow, NS, mc, row_ptr, pre, epi, wait, tid, wave, lane);
+        down_tiles<2>(a, L, wrow0, row0, mc, n, wait, wave, tid, lane);
 }
 
 constexpr uint64_t kPfWaitTicks = 20000000;  // 200 ms of the 100 MHz wall clock
@@ -940,16 +924,16 @@ constexpr uint64_t kPfWaitTicks = 20000000;  // 200 ms of the 100 MHz wall clock
 }  // namespace
 
 template <int ACT>
-__global__ void __launch_bounds__(256, 2) k_prefill_gate_up(PfArgs a) {
-    __shared__ __attribute__((aligned(16))) _Float16 Bs[2][NB][LDK];
-    gate_up_body<ACT>(a, blockIdx.x, blockIdx.y, Bs);
+__global__ void __launch_bounds__(PT, 4) k_prefill_gate_up(PfArgs a) {
+    __shared__ GemmLds L;
+    gate_up_body<ACT>(a, blockIdx.x, blockIdx.y, L);
 }
 
 // ---------------------------------------------------------------- down
-__global__ void __launch_bounds__(256, 2) k_prefill_down(PfArgs a) {
+__global__ void __launch_bounds__(PT, 4) k_prefill_down(PfArgs a) {
     if ((int)blockIdx.y >= *a.n_chunks) return;
-    __shared__ __attribute__((aligned(16))) _Float16 Bs[2][NB][LDK];
-    down_body(a, blockIdx.x, blockIdx.y, Bs, NoWait{});
+    __shared__ GemmLds L;
+    down_body(a, blockIdx.x, blockIdx.y, L, NoWait{});
 }
 
 // ---------------------------------------------------------------- both GEMMs in one launch
@@ -967,13 +951,13 @@ __global__ void __launch_bounds__(256, 2) k_prefill_down(PfArgs a) {
 // dispatched first; the wait is bounded by the wall clock (on expiry the
 // error word is set and that call's outputs are wrong).
 template <int ACT>
-__global__ void __launch_bounds__(256, 2) k_prefill_gemms(PfArgs a) {
-    __shared__ __attribute__((aligned(16))) _Float16 Bs[2][NB][LDK];
+__global__ void __launch_bounds__(PT, 4) k_prefill_gemms(PfArgs a) {
+    __shared__ GemmLds L;
     const int g = blockIdx.x & 7, s = blockIdx.x >> 3;
     const int ngx = a.F / BN1, ngu = ngx * a.CG;
     if (s < ngu) {
         const int y = g + 8 * (s / ngx);
-        if (!gate_up_body<ACT>(a, s % ngx, y, Bs)) return;
+        if (!gate_up_body<ACT>(a, s % ngx, y, L)) return;
         // every thread's H stores acknowledged by the L2 before the count
         asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
         __syncthreads();
@@ -999,7 +983,7 @@ __global__ void __launch_bounds__(256, 2) k_prefill_gemms(PfArgs a) {
         }
         __syncthreads();
     };
-    down_body(a, s2 % ndx, y, Bs, wait);
+    down_body(a, s2 % ndx, y, L, wait);
 }
 
 // ---------------------------------------------------------------- combine
@@ -1042,7 +1026,7 @@ __global__ void __launch_bounds__(256) k_prefill_combine(const float *__restrict
 
 size_t prefill_workspace_bytes(int T, int k, int E, int Kd, int D) {
     const size_t TK = (size_t)T * k;
-    return align256((size_t)T * E * 4) + 2 * align256(TK * 4) + align256((size_t)(E + 1) * 4) +
+    return align256((size_t)T * E * 4) + 2 * align256(TK * 4) +
            align256((size_t)max_chunks((int)TK, E) * 12) + 256 + 2 * align256(TK * 4) + align256((size_t)T * 4) +
            align256((size_t)T * D * 2) + align256(TK * Kd * 2) + align256(TK * D * 4) +
            align256((size_t)max_chunks((int)TK, E) * 4);
@@ -1058,8 +1042,8 @@ hipError_t launch_moe_prefill(const DevTensor &R, const DevTensor &GU, const Dev
     hipError_t e = launch_router_batched(R, X, T, bias, w.logits, k, norm, w.ids, w.w, w.Xh, w.rs, &x_done, s);
     if (e != hipSuccess) return e;
     const int mc = max_chunks(TK, E);
-    hipLaunchKernelGGL(k_prefill_dispatch, dim3(1), dim3(1024), 0, s, w.ids, TK, k, E, w.offsets, w.chunks,
-                       w.n_chunks, w.perm, w.pos, w.done, mc);
+    hipLaunchKernelGGL(k_prefill_dispatch, dim3(1), dim3(1024), 0, s, w.ids, TK, k, E, w.chunks, w.n_chunks,
+                       w.perm, w.pos, w.done, mc);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (!x_done) {
         hipLaunchKernelGGL(k_prefill_x_f16, dim3((unsigned)T), dim3(256), 0, s, X, w.Xh, w.rs, D);
@@ -1075,7 +1059,6 @@ hipError_t launch_moe_prefill(const DevTensor &R, const DevTensor &GU, const Dev
     pa.D = D;
     pa.chunks = w.chunks;
     pa.n_chunks = w.n_chunks;
-    pa.offsets = w.offsets;
     pa.perm = w.perm;
     pa.H = w.H;
     pa.Kd = Kd;
@@ -1089,15 +1072,30 @@ hipError_t launch_moe_prefill(const DevTensor &R, const DevTensor &GU, const Dev
     pa.X = X;
     // (LT_PREFILL_NO_TINY, read at each call: every chunk on the tiles, for testing)
     pa.tiny = GU.blocks_per_row <= 8 && Dn.blocks_per_row <= 4 && !getenv("LT_PREFILL_NO_TINY");
+    const int ngx = F / BN1, ndx = D / BN2;
     if (xcd_local) {
-        const unsigned nb = 8u * (unsigned)((F / BN1 + D / BN2) * pa.CG);
-        hipLaunchKernelGGL(act == 1u ? k_prefill_gemms<1> : k_prefill_gemms<0>, dim3(nb), dim3(256), 0, s, pa);
+        // Blocks a CU: four, or two (16 KB more LDS a block) where the gate/up
+        // blocks to be expected -- a chunk per MC rows and one more for half
+        // of the experts -- leave places free at four a CU.  Down blocks of
+        // unfinished chunks would take those places, each fixed to the CU it
+        // waits on, and what they then draw from memory delays the gate/up
+        // blocks beside them that others still wait for.  Whole calls, four |
+        // two a CU, 2048 x 768, 128 experts, 8 a token, routing as skewed as
+        // a text's: 8 tokens 67 | 62 us, 37 92 | 71, 100 109 | 85, 200 101 |
+        // 106, 512 143 | 161, 1024 219 | 242; 1000 tokens of 1280 x 448, 32
+        // experts, 4 a token: 113 | 85.  (Even routings, with a chunk for
+        // every expert, turn earlier: 64 tokens 108 | 121, but the host does
+        // not know them.)
+        const unsigned nb = 8u * (unsigned)((ngx + ndx) * pa.CG);
+        const bool two = (TK / MC + min(E, TK) / 2) * ngx < 4 * 256;
+        hipLaunchKernelGGL(act == 1u ? k_prefill_gemms<1> : k_prefill_gemms<0>, dim3(nb), dim3(PT), two ? 16384 : 0, s,
+                           pa);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     } else {
-        hipLaunchKernelGGL(act == 1u ? k_prefill_gate_up<1> : k_prefill_gate_up<0>, dim3(F / BN1, mc), dim3(256), 0,
-                           s, pa);
+        hipLaunchKernelGGL(act == 1u ? k_prefill_gate_up<1> : k_prefill_gate_up<0>, dim3(ngx, mc), dim3(PT), 0, s,
+                           pa);
         if ((e = hipGetLastError()) != hipSuccess) return e;
-        hipLaunchKernelGGL(k_prefill_down, dim3(D / BN2, mc), dim3(256), 0, s, pa);
+        hipLaunchKernelGGL(k_prefill_down, dim3(ndx, mc), dim3(PT), 0, s, pa);
         if ((e = hipGetLastError()) != hipSuccess) return e;
     }
     hipLaunchKernelGGL(k_prefill_combine, dim3((D / 4 + 255) / 256, T), dim3(256), 0, s, w.Y, w.pos, w.w, w.rs, k, D,

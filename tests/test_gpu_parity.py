@@ -1015,6 +1015,28 @@ def test_gpu_prefill_many_placement_tables(ctx, pool, T, E, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("D,F", [(256, 64), (1280, 320), (2304, 1088)])  # 1, 5, 9 and 1, 2, 5 super-blocks a row
+def test_gpu_prefill_chunk_edges(ctx, pool, D, F):
+    # two experts that every token takes: an expert's rows are the batch's,
+    # around the edges of a token tile (32 rows) and of a chunk (64); one
+    # expert row wrong or missing is past the bound by an order
+    w = synth.moe_weights(87, D, 2, F, down_cols=(F + 255) // 256 * 256)
+    router, gate_up, down = lt.upload_moe(ctx, w)
+    X = synth.normal(synth.stream(88, D), (129, D))
+    ref, rids, _ = orc.moe_prefill(w, X, 2, norm_topk=True, pool=pool)
+    for T in (1, 31, 32, 33, 63, 64, 65, 96, 97, 128, 129):
+        out = np.full((T, D), np.nan, np.float32)
+        ids = np.zeros((T, 2), np.uint32)
+        ctx.moe_prefill(out, X[:T], router, gate_up, down, 2, F, norm_topk=True, out_ids=ids)
+        assert np.array_equal(ids, rids[:T])
+        err = np.linalg.norm(out - ref[:T], axis=1) / np.linalg.norm(ref[:T], axis=1)
+        assert err.max() <= 2 * PREFILL_REL_L2, (T, int(err.argmax()), float(err.max()))  # (single rows)
+        assert rel_l2(out, ref[:T]) <= PREFILL_REL_L2, T
+    for t in (router, gate_up, down):
+        t.free()
+
+
+@pytest.mark.gpu
 def test_gpu_prefill_one_token_chunks(ctx, cfg3, pool):
     # experts that get one token of the batch stream their weights against
     # the token's int8 limbs instead of an f16 tile; LT_PREFILL_NO_TINY
