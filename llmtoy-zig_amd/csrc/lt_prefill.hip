@@ -4,10 +4,10 @@
 // (main.zig:1916-1922).  Here T tokens go through the layer together:
 //   1. router logits for all tokens with the reference's exact dotf32 order
 //      and per-token softmax / top-k (lt_router.hip);
-//   2. dispatch: one block counts tokens per expert, lays out per-expert
-//      row ranges ("sorted rows"), cuts each range into chunks of at most
-//      MC = 64 rows, and places the (token, slot) assignments into them in
-//      assignment order (a stable counting sort);
+//   2. dispatch: a block per expert lays its rows out behind those of the
+//      experts before it ("sorted rows"), cuts them into chunks of at most
+//      MC = 64, and places its (token, slot) assignments in assignment order
+//      (a stable counting sort);
 //      X is converted to f16 once (by the router kernel, or
 //      k_prefill_x_f16), each row t divided by r_t = 2^e, a power of two
 //      that puts its largest element in [1, 2);
@@ -317,223 +317,112 @@ __device__ __forceinline__ void gemm_tiles(floatx16 (&acc)[MT], GemmLds &L, cons
 }  // namespace
 
 // ---------------------------------------------------------------- dispatch
-// The lanes of the wavefront whose id equals this lane's (ids below 2^nb,
-// invalid ids >= E in a group of their own): one ballot per id bit.
-__device__ __forceinline__ uint64_t match_ids(uint32_t x, bool valid, int nb) {
-    uint64_t m = __ballot(1);  // the active lanes
-    const uint64_t v = __ballot(valid);
-    m &= valid ? v : ~v;
-    for (int b = 0; b < nb; b++) {
-        const bool on = (x >> b) & 1u;
-        const uint64_t bb = __ballot(on);
-        m &= on ? bb : ~bb;
-    }
-    return m;
-}
-
 // Lanes of m below this lane.
 __device__ __forceinline__ int rank_in(uint64_t m) {
     return (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
 }
 
-// One block of 1024 threads.  Assignment i = t k + s goes to sorted row
-// offsets[e] + (the number of assignments before i with the same expert e):
-// a stable counting sort, so every row's chunk, and with it the row's
-// result (the chunk's token tiles pick the GEMM's K split), is the same on
-// every call.  Assignments are taken in rounds of 1024 (i = 1024 r + tid),
-// a round in 16 segments of 64 (its wavefronts).  Within a wavefront the
-// lanes with equal ids find each other with one ballot per id bit
-// (match_ids); the first lane of each group adds the group's size to its
-// expert's count and, for the placement, writes it to the segment's entry
-// of a [segment][expert] table, which P = 1024 / E threads per expert
-// turn into each segment's first row (an exclusive scan over segments, the
-// experts' running rows carried from one batch of rounds to the next).
-// Per expert e (thread e): v[0] = its row count, v[1] = its full chunks,
-// v[2 + c] = 1 if its last chunk is partial with c + 1 token tiles.  An
-// inclusive scan over experts (wavefront scans, then the wavefront totals)
-// gives every expert its row offset and the positions of its chunks in a
-// list ordered by token tiles, largest first: the blocks with the most
-// MFMA work are dispatched first and the short ones fill in behind them.
-// Up to kIdsPer ids per thread are loaded once, all in flight together,
-// and kept with their ranks for the placement; longer batches read them
+// Block e places expert e's assignments: assignment i = t k + s goes to sorted
+// row (number of valid ids below e) + (number of assignments before i with
+// the same expert), a stable counting sort, so every row's chunk is the same
+// on every call.  Wavefront w takes assignments [w seg, (w + 1) seg), 64 at a
+// time: the lanes that hold e find their ranks with one ballot, and the
+// wavefronts' totals meet in LDS.  Every block counts all experts as well (LDS
+// atomics; a token's k experts are distinct, so few lanes share a counter),
+// because a chunk's place in the list depends on all of them: full chunks in
+// expert order first, then the partial ones of two token tiles, then of one
+// -- the blocks with the most MFMA work are dispatched first and the short
+// ones fill in behind them.  Each wavefront sums the counters for itself, so
+// the counters' barrier is the only one behind the loads.  Up to kIds ids per
+// lane are loaded once, all in flight together; longer batches read them
 // again.
-__global__ void __launch_bounds__(1024) k_prefill_dispatch(const uint32_t *__restrict__ ids, int TK, int k, int E,
-                                                           int *__restrict__ chunks, int *__restrict__ n_chunks,
-                                                           int *__restrict__ perm,
-                                                           int *__restrict__ pos, int *__restrict__ done, int maxc) {
-    constexpr int kIdsPer = 8, kTab = 16384;
-    __shared__ int cnt[1024], cur[1024], psum[1024];
-    __shared__ int tab[kTab];  // [segment][E]: group sizes, then the segment's first rows
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const int nb = E > 1 ? 32 - __builtin_clz((unsigned)(E - 1)) : 0;
-    const bool cached = TK <= kIdsPer * 1024;
-    const int rounds = (TK + 1023) / 1024;
-    uint32_t xc[kIdsPer];
-    int rk[kIdsPer], gs[kIdsPer];  // cached: rank in the wavefront's group, group size (0: not the group's first)
+// Bound: the latency of the chain ids -> counters -> sums -> rows.  One block
+// that sorted for all experts (a table of group sizes per 64 assignments and
+// expert) took 6.4, 10.6 and 15.6 us for 37, 512 and 1024 tokens of 8 experts
+// each out of 128, a block per expert 4.6, 7.0 and 10.2 us.
+__global__ void __launch_bounds__(512) k_prefill_dispatch(const uint32_t *__restrict__ ids, int TK, int k, int E,
+                                                          int *__restrict__ chunks, int *__restrict__ n_chunks,
+                                                          int *__restrict__ perm, int *__restrict__ pos,
+                                                          int *__restrict__ done, int maxc) {
+    constexpr int kIds = 16, kWaves = 8;
+    __shared__ int cnt[1024], own[kWaves];
+    const int e = blockIdx.x, tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int seg = (TK + 64 * kWaves - 1) / (64 * kWaves) * 64;
+    const int i0 = wave * seg + lane, nj = seg / 64;  // this lane's assignments: i0 + 64 j, j < nj
+    const bool cached = nj <= kIds;
+    // i / k = i per_k / 2^31 for the i < 2^20 and k <= 16 there are: per_k k - 2^31 < k, and i k < 2^31
+    const uint32_t per_k = ((1u << 31) + (uint32_t)k - 1) / (uint32_t)k;
+    uint32_t xc[kIds];
+    if (cached) {
 #pragma unroll
-    for (int j = 0; j < kIdsPer; j++) {
-        const int i = tid + j * 1024;
-        xc[j] = cached && i < TK ? ids[i] : 0xffffffffu;
+        for (int j = 0; j < kIds; j++) xc[j] = j < nj && i0 + 64 * j < TK ? ids[i0 + 64 * j] : 0xffffffffu;
     }
-    // placement in batches of RB rounds (16 RB segments x E in the table)
-    const int RB = max(1, min(kIdsPer, kTab / (16 * E)));
-    if (tid < E) cnt[tid] = 0;
-    for (int i = tid; i < maxc; i += 1024) done[i] = 0;  // the fused GEMMs' per-chunk counts
-    for (int q = tid; q < 16 * min(RB, rounds) * E; q += 1024) tab[q] = 0;  // (the first batch's table)
+    for (int q = tid; q < E; q += 512) cnt[q] = 0;
+    for (int i = e * 512 + tid; i < maxc; i += 512 * E) done[i] = 0;  // the fused GEMMs' per-chunk counts
     __syncthreads();
-    auto group = [&](uint32_t x, int &rank, int &size) {
-        const bool valid = x < (uint32_t)E;
-        const uint64_t m = match_ids(x, valid, nb);
-        rank = rank_in(m);
-        size = valid && rank == 0 ? __popcll(m) : 0;
-    };
-    // assignment tid + 1024 r: id, rank, group size
-    auto get = [&](int r, uint32_t &x, int &rank, int &size) {
-        if (cached) {
-            x = 0xffffffffu;
-            rank = size = 0;
-#pragma unroll
-            for (int j = 0; j < kIdsPer; j++)
-                if (j == r) {
-                    x = xc[j];
-                    rank = rk[j];
-                    size = gs[j];
-                }
-        } else {
-            const int i = tid + 1024 * r;
-            x = i < TK ? ids[i] : 0xffffffffu;
-            group(x, rank, size);
-        }
+    int mine = 0;  // (the wavefront's)
+    auto count = [&](uint32_t x) {
+        if (x < (uint32_t)E) atomicAdd(&cnt[x], 1);
+        mine += __popcll(__ballot(x == (uint32_t)e));
     };
     if (cached) {
 #pragma unroll
-        for (int j = 0; j < kIdsPer; j++) {
-            if (j < rounds) {
-                group(xc[j], rk[j], gs[j]);
-                if (gs[j]) atomicAdd(&cnt[xc[j]], gs[j]);
-            }
-        }
+        for (int j = 0; j < kIds; j++)
+            if (j < nj) count(xc[j]);
     } else {
-        for (int i = tid; i < TK; i += 1024) {
-            const uint32_t x = ids[i];
-            if (x < (uint32_t)E) atomicAdd(&cnt[x], 1);
-        }
+#pragma unroll 8
+        for (int j = 0; j < nj; j++) count(i0 + 64 * j < TK ? ids[i0 + 64 * j] : 0xffffffffu);
     }
+    if (lane == 0) own[wave] = mine;
     __syncthreads();
-    // Experts in order, by wavefront 0: lane l takes experts CH l + [0, CH)
-    // (CH = ceil(E / 64)); the lanes' totals of rows, full chunks and
-    // partial chunks of each tile count (two 16-bit counts per word) are
-    // scanned over the lanes, then each lane lays out its experts' rows and
-    // chunks -- full chunks first, then the partial ones by token tiles,
-    // largest first: the blocks with the most MFMA work are dispatched
-    // first and the short ones fill in behind them.
-    if (wave == 0) {
-        const int CH = (E + 63) >> 6;
-        int t0 = 0, t1 = 0, t12 = 0;  // rows, full chunks, partial chunks of 1 | 2 << 16 tiles
-        for (int q = 0; q < CH; q++) {
-            const int e = CH * lane + q;
-            const int n = e < E ? cnt[e] : 0, rem = n % MC, cls = rem ? (rem + 31) / 32 : 0;
-            t0 += n;
-            t1 += n / MC;
-            t12 += (cls == 1 ? 1 : 0) + (cls == 2 ? 0x10000 : 0);
-        }
-        int i0 = t0, i1 = t1, i12 = t12;  // inclusive scans over the lanes
-#pragma unroll
-        for (int d = 1; d < 64; d <<= 1) {
-            const int a0 = __shfl_up(i0, d, 64), a1 = __shfl_up(i1, d, 64);
-            const int a12 = __shfl_up(i12, d, 64);
-            if (lane >= d) {
-                i0 += a0;
-                i1 += a1;
-                i12 += a12;
-            }
-        }
-        const int tot_full = __shfl(i1, 63, 64), T12 = __shfl(i12, 63, 64);
-        const int tot_p2 = T12 >> 16, tot_p1 = T12 & 0xffff;
-        // first chunk index of each partial class, then this lane's running positions
-        int off = i0 - t0, fc = i1 - t1;
-        int pc[2] = {tot_full + tot_p2 + ((i12 - t12) & 0xffff), tot_full + ((i12 - t12) >> 16)};
-        for (int q = 0; q < CH; q++) {
-            const int e = CH * lane + q;
-            if (e >= E) break;
-            const int n = cnt[e], full = n / MC, rem = n % MC, cls = rem ? (rem + 31) / 32 : 0;
-            cur[e] = off;
-            for (int j = 0; j < full; j++) {
-                int *ch = chunks + 3 * (fc + j);
-                ch[0] = e;
-                ch[1] = off + j * MC;
-                ch[2] = MC;
-            }
-            fc += full;
-            if (cls) {
-                int *ch = chunks + 3 * pc[cls - 1];
-                ch[0] = e;
-                ch[1] = off + full * MC;
-                ch[2] = rem;
-                pc[cls - 1]++;
-            }
-            off += n;
-            if (e == E - 1) *n_chunks = tot_full + tot_p2 + tot_p1;
-        }
+    // rows below e, and the chunks of each kind (full, partial of two tiles, of
+    // one): those below e in the low half, all of them in the high half
+    int rows = 0, full = 0, two = 0, one = 0;
+    for (int q = lane; q < E; q += 64) {
+        const int n = cnt[q], rem = n % MC, f = q < e ? 0x10001 : 0x10000;
+        rows += q < e ? n : 0;
+        full += n / MC * f;
+        two += rem > 32 ? f : 0;
+        one += rem > 0 && rem <= 32 ? f : 0;
     }
-    __syncthreads();
-    // placement: cur[e] = the expert's next free row
-    const int P = min(32, 1024 / E), pe = tid % E, pp = tid / E;  // thread pp < P of expert pe
-    for (int r0 = 0; r0 < rounds; r0 += RB) {
-        const int nr = min(RB, rounds - r0), SB = 16 * nr;
-        uint32_t xb[kIdsPer];
-        int rkb[kIdsPer];
-        if (r0 > 0) {  // (the first batch's table was cleared at the start)
-            __syncthreads();  // the previous batch's reads of the table are done
-            for (int q = tid; q < SB * E; q += 1024) tab[q] = 0;
-            __syncthreads();
-        }
 #pragma unroll
-        for (int rr = 0; rr < kIdsPer; rr++) {
-            if (rr < nr) {
-                int size;
-                get(r0 + rr, xb[rr], rkb[rr], size);
-                if (size) tab[(16 * rr + wave) * E + xb[rr]] = size;
-            }
-        }
-        __syncthreads();
-        const int SP = (SB + P - 1) / P, s0 = pp * SP, s1 = min(SB, s0 + SP);
-        if (pp < P) {
-            int loc = 0;
-            for (int sg = s0; sg < s1; sg++) loc += tab[sg * E + pe];
-            psum[pp * E + pe] = loc;
-        }
-        __syncthreads();
-        int total = 0;
-        if (pp < P) {
-            int base = cur[pe];
-            for (int p2 = 0; p2 < P; p2++) {
-                const int ps = psum[p2 * E + pe];
-                base += p2 < pp ? ps : 0;
-                total += ps;
-            }
-            for (int sg = s0; sg < s1; sg++) {
-                const int c = tab[sg * E + pe];
-                tab[sg * E + pe] = base;
-                base += c;
-            }
-        }
-        __syncthreads();
-        if (pp == 0) cur[pe] += total;  // (read again only after the next batch's first barrier)
+    for (int d = 1; d < 64; d <<= 1) {
+        rows += __shfl_xor(rows, d, 64);
+        full += __shfl_xor(full, d, 64);
+        two += __shfl_xor(two, d, 64);
+        one += __shfl_xor(one, d, 64);
+    }
+    const int tot_full = full >> 16, tot_two = two >> 16, n = cnt[e], nf = n / MC, rem = n % MC;
+    if (e == 0 && tid == 0) *n_chunks = tot_full + tot_two + (one >> 16);
+    for (int c = tid; c < nf + (rem ? 1 : 0); c += 512) {
+        const int at = c < nf      ? (full & 0xffff) + c
+                       : rem > 32 ? tot_full + (two & 0xffff)
+                                  : tot_full + tot_two + (one & 0xffff);
+        chunks[3 * at] = e;
+        chunks[3 * at + 1] = rows + c * MC;
+        chunks[3 * at + 2] = c < nf ? MC : rem;
+    }
+    int row = rows;
 #pragma unroll
-        for (int rr = 0; rr < kIdsPer; rr++) {
-            const int i = tid + 1024 * (r0 + rr);
-            if (rr < nr && i < TK) {
-                const uint32_t x = xb[rr];
-                if (x < (uint32_t)E) {
-                    const int p = tab[(16 * rr + wave) * E + x] + rkb[rr];
-                    perm[p] = i / k;
-                    pos[i] = p;
-                } else {
-                    pos[i] = -1;
-                }
-            }
+    for (int w = 0; w < kWaves; w++) row += w < wave ? own[w] : 0;
+    auto place = [&](uint32_t x, int i) {
+        const uint64_t m = __ballot(x == (uint32_t)e);
+        if (x == (uint32_t)e) {
+            const int p = row + rank_in(m);
+            perm[p] = (int)((uint64_t)i * per_k >> 31);
+            pos[i] = p;
+        } else if (e == 0 && x >= (uint32_t)E && i < TK) {
+            pos[i] = -1;  // (no expert: the combine leaves the slot out)
         }
+        row += __popcll(m);
+    };
+    if (cached) {
+#pragma unroll
+        for (int j = 0; j < kIds; j++)
+            if (j < nj) place(xc[j], i0 + 64 * j);
+    } else {
+#pragma unroll 8
+        for (int j = 0; j < nj; j++) place(i0 + 64 * j < TK ? ids[i0 + 64 * j] : 0xffffffffu, i0 + 64 * j);
     }
 }
 
@@ -1042,7 +931,7 @@ hipError_t launch_moe_prefill(const DevTensor &R, const DevTensor &GU, const Dev
     hipError_t e = launch_router_batched(R, X, T, bias, w.logits, k, norm, w.ids, w.w, w.Xh, w.rs, &x_done, s);
     if (e != hipSuccess) return e;
     const int mc = max_chunks(TK, E);
-    hipLaunchKernelGGL(k_prefill_dispatch, dim3(1), dim3(1024), 0, s, w.ids, TK, k, E, w.chunks, w.n_chunks,
+    hipLaunchKernelGGL(k_prefill_dispatch, dim3(E), dim3(512), 0, s, w.ids, TK, k, E, w.chunks, w.n_chunks,
                        w.perm, w.pos, w.done, mc);
     if ((e = hipGetLastError()) != hipSuccess) return e;
     if (!x_done) {

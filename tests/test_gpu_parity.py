@@ -1015,6 +1015,25 @@ def test_gpu_prefill_many_placement_tables(ctx, pool, T, E, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,k", [(1, 1, 1), (513, 3, 1), (1024, 128, 8), (8193, 5, 1), (70, 1024, 16)])
+def test_gpu_prefill_dispatch_edges(ctx, pool, T, E, k):
+    # the placement, a block per expert: one assignment, a wavefront's share
+    # that ends inside its 64 lanes, the most ids that stay in registers
+    # (8,192) and one more, the most experts
+    w = synth.moe_weights(89, 256, E, 64, down_cols=256)
+    router, gate_up, down = lt.upload_moe(ctx, w)
+    X = synth.normal(synth.stream(90, T), (T, 256))
+    out = np.full((T, 256), np.nan, np.float32)
+    ctx.moe_prefill(out, X, router, gate_up, down, k, 64, norm_topk=True)
+    sel = np.unique(np.r_[np.arange(0, T, max(1, T // 60)), T - 1])
+    ref, _, _ = orc.moe_prefill(w, X[sel], k, norm_topk=True, pool=pool)
+    assert np.isfinite(out).all()
+    assert rel_l2(out[sel], ref) <= PREFILL_REL_L2
+    for t in (router, gate_up, down):
+        t.free()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("D,F", [(256, 64), (1280, 320), (2304, 1088)])  # 1, 5, 9 and 1, 2, 5 super-blocks a row
 def test_gpu_prefill_chunk_edges(ctx, pool, D, F):
     # two experts that every token takes: an expert's rows are the batch's,
