@@ -369,12 +369,12 @@ hipError_t launch_router(const DevTensor &R, const float *x, const float *bias, 
 
 // Batched F32 router (prefill): block = RB router rows x TB tokens.  Thread
 // (c = tid % 32, g = tid / 32) runs dotf32 chain c (elements 32 it + c) of
-// 4 rows x 4 tokens side by side -- the same rounded products and adds in
-// the same order per chain as k_router_f32, so the logits are identical --
-// with K staged through LDS 256 at a time (double-buffered) and each loaded
-// value used by 4 chains.  The 32 chain totals of a (row, token) then meet
-// in LDS for the (acc0+acc1)+(acc2+acc3) and ordered lane reduce.
-// Requires cols % 256 == 0.
+// RB / 2 rows x TB / 4 tokens side by side -- the same rounded products and
+// adds in the same order per chain as k_router_f32, so the logits are
+// identical -- with K staged through LDS KC at a time (double-buffered,
+// loads P stages ahead in registers) and each loaded value used by several
+// chains.  The 32 chain totals of a (row, token) then meet in LDS for the
+// (acc0+acc1)+(acc2+acc3) and ordered lane reduce.  Requires cols % 256 == 0.
 // With Xh set, the same launch writes the prefill's f16 X (Xh, row scales
 // rs; prefill_x_exp / prefill_x_store8): token t0 + j of the tile is
 // converted by wavefront w of the row block with j = blockIdx.x + gridDim.x
@@ -383,95 +383,95 @@ hipError_t launch_router(const DevTensor &R, const float *x, const float *bias, 
 // tile as well, behind an arrival ticket, made the launch 70 us instead of
 // 15: the release fences of 512 blocks write back the L2s the f16 rows have
 // filled.)
-constexpr int RT_RB = 8, RT_TB = 16, RT_KC = 256;
-
+// Bound: large batches by the vector unit (a product and an add a term, kept
+// apart for the order), so an 8 x 16 tile shares each LDS value four times and
+// its 24 KB let all blocks of a 1024-token call be resident; small ones by
+// one wavefront's chain of instructions, so a 4 x 8 tile with a quarter of
+// them and four stages of loads in flight.
+// 128 rows of 2,048, us for 37 | 512 | 1024 tokens: 8 x 16 tiles with 256 of K
+// a stage, one stage of loads ahead, 11.0 | 15.0 | 28.3; <8, 16, 128, 2> 12.1 |
+// 15.6 | 24.0; <4, 8, 256, 4> 7.5 | 22.5 | 38.5.
+template <int RB, int TB, int KC, int P>
 __global__ void __launch_bounds__(256) k_router_f32_tile(const float *__restrict__ W, const float *__restrict__ X,
                                                          const float *__restrict__ bias, float *__restrict__ logits,
                                                          int rows, int cols, int T, _Float16 *__restrict__ Xh,
                                                          float *__restrict__ rs) {
 #pragma clang fp contract(off)
-    __shared__ __attribute__((aligned(16))) float ws[2][RT_RB][RT_KC];
-    __shared__ __attribute__((aligned(16))) float xs[2][RT_TB][RT_KC];
-    __shared__ float ch[RT_RB][RT_TB][33];
+    constexpr int RI = RB / 2, TJ = TB / 4, R4 = KC / 4, NU = (RB + TB) * R4 / 256;
+    static_assert((RB + TB) * R4 % 256 == 0 && P % 2 == 0, "whole loads, static buffers");
+    static_assert(RB * TB * 33 <= 2 * (RB + TB) * KC, "the chain totals take the tiles' place");
+    __shared__ __attribute__((aligned(16))) float tile[2][RB + TB][KC];  // router rows, then tokens
     const int tid = threadIdx.x, c = tid & 31, g = tid >> 5;
     const int wave = tid >> 6, lane = tid & 63;
-    const int rg = g & 1, tg = g >> 1;  // rows 4 rg + [0, 4), tokens 4 tg + [0, 4)
-    const int r0 = blockIdx.x * RT_RB, t0 = blockIdx.y * RT_TB;
+    const int rg = g & 1, tg = g >> 1;  // rows RI rg + [0, RI), tokens TJ tg + [0, TJ)
+    const int r0 = blockIdx.x * RB, t0 = blockIdx.y * TB;
     // this wavefront's token for the f16 X (uniform over the wavefront)
     const int xj = blockIdx.x + gridDim.x * wave;
-    const bool xconv = Xh && xj < RT_TB && t0 + xj < T;
+    const bool xconv = Xh && xj < TB && t0 + xj < T;
     float xmax = 0.0f;
-    // stage loads: W tile 8 x 256 = 512 float4 (2 per thread), X tile
-    // 16 x 256 = 1024 float4 (4 per thread); rows / tokens past the end
-    // re-read the last valid one (never used)
-    const float *wsrc[2], *xsrc[4];
+    // a stage's NU float4 of this thread; rows / tokens past the end re-read
+    // the last valid one (never used)
+    const float *src[NU];
 #pragma unroll
-    for (int u = 0; u < 2; u++) {
-        const int f = tid + 256 * u, r = f >> 6;
-        wsrc[u] = W + (size_t)min(r0 + r, rows - 1) * cols + (f & 63) * 4;
+    for (int u = 0; u < NU; u++) {
+        const int f = tid + 256 * u, r = f / R4;
+        src[u] = (r < RB ? W + (size_t)min(r0 + r, rows - 1) * cols : X + (size_t)min(t0 + r - RB, T - 1) * cols) +
+                 (f % R4) * 4;
     }
+    const int nkc = cols / KC;
+    float4 v[P][NU];
 #pragma unroll
-    for (int u = 0; u < 4; u++) {
-        const int f = tid + 256 * u, t = f >> 6;
-        xsrc[u] = X + (size_t)min(t0 + t, T - 1) * cols + (f & 63) * 4;
-    }
-    float4 wr[2], xr[4];
+    for (int p = 0; p < P; p++)
 #pragma unroll
-    for (int u = 0; u < 2; u++) wr[u] = ldg16f(wsrc[u]);
+        for (int u = 0; u < NU; u++) v[p][u] = ldg16f(src[u] + min(p, nkc - 1) * KC);
+    float acc[RI][TJ];
 #pragma unroll
-    for (int u = 0; u < 4; u++) xr[u] = ldg16f(xsrc[u]);
-    float acc[4][4];
+    for (int i = 0; i < RI; i++)
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+        for (int j = 0; j < TJ; j++) acc[i][j] = 0.0f;
+    auto stage = [&](float4 (&q)[NU], int kc, int b) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) acc[i][j] = 0.0f;
-    const int nkc = cols / RT_KC;
-    for (int kc = 0; kc < nkc; kc++) {
-        const int b = kc & 1;
-#pragma unroll
-        for (int u = 0; u < 2; u++) {
+        for (int u = 0; u < NU; u++) {
             const int f = tid + 256 * u;
-            *reinterpret_cast<float4 *>(&ws[b][f >> 6][(f & 63) * 4]) = wr[u];
-        }
-#pragma unroll
-        for (int u = 0; u < 4; u++) {
-            const int f = tid + 256 * u;
-            *reinterpret_cast<float4 *>(&xs[b][f >> 6][(f & 63) * 4]) = xr[u];
+            *reinterpret_cast<float4 *>(&tile[b][f / R4][(f % R4) * 4]) = q[u];
         }
         __syncthreads();
-        if (kc + 1 < nkc) {  // next chunk's loads in flight during this one
 #pragma unroll
-            for (int u = 0; u < 2; u++) wr[u] = ldg16f(wsrc[u] + (kc + 1) * RT_KC);
-#pragma unroll
-            for (int u = 0; u < 4; u++) xr[u] = ldg16f(xsrc[u] + (kc + 1) * RT_KC);
-        }
+        for (int u = 0; u < NU; u++) q[u] = ldg16f(src[u] + min(kc + P, nkc - 1) * KC);
         if (xconv) {
-            const float4 v = *reinterpret_cast<const float4 *>(&xs[b][xj][4 * lane]);
-            xmax = fmaxf(xmax, fmaxf(fmaxf(fabsf(v.x), fabsf(v.y)), fmaxf(fabsf(v.z), fabsf(v.w))));
+            const float4 x = *reinterpret_cast<const float4 *>(&tile[b][RB + xj][4 * (lane % R4)]);
+            xmax = fmaxf(xmax, fmaxf(fmaxf(fabsf(x.x), fabsf(x.y)), fmaxf(fabsf(x.z), fabsf(x.w))));
         }
 #pragma unroll
-        for (int it = 0; it < RT_KC / 32; it++) {
-            float wv[4], xv[4];
+        for (int it = 0; it < KC / 32; it++) {
+            float wv[RI], xv[TJ];
 #pragma unroll
-            for (int i = 0; i < 4; i++) wv[i] = ws[b][4 * rg + i][it * 32 + c];
+            for (int i = 0; i < RI; i++) wv[i] = tile[b][RI * rg + i][it * 32 + c];
 #pragma unroll
-            for (int j = 0; j < 4; j++) xv[j] = xs[b][4 * tg + j][it * 32 + c];
+            for (int j = 0; j < TJ; j++) xv[j] = tile[b][RB + TJ * tg + j][it * 32 + c];
 #pragma unroll
-            for (int i = 0; i < 4; i++)
+            for (int i = 0; i < RI; i++)
 #pragma unroll
-                for (int j = 0; j < 4; j++) {
+                for (int j = 0; j < TJ; j++) {
                     const float p = wv[i] * xv[j];
                     acc[i][j] = acc[i][j] + p;
                 }
         }
+    };
+    for (int kc = 0; kc < nkc; kc += P) {
+#pragma unroll
+        for (int p = 0; p < P; p++)
+            if (kc + p < nkc) stage(v[p], kc + p, p & 1);
     }
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) ch[4 * rg + i][4 * tg + j][c] = acc[i][j];
     __syncthreads();
-    if (tid < RT_RB * RT_TB) {
-        const int r = tid / RT_TB, t = tid % RT_TB, row = r0 + r, tok = t0 + t;
+    float(*const ch)[TB][33] = reinterpret_cast<float(*)[TB][33]>(&tile[0][0][0]);
+#pragma unroll
+    for (int i = 0; i < RI; i++)
+#pragma unroll
+        for (int j = 0; j < TJ; j++) ch[RI * rg + i][TJ * tg + j][c] = acc[i][j];
+    __syncthreads();
+    if (tid < RB * TB) {
+        const int r = tid / TB, t = tid % TB, row = r0 + r, tok = t0 + t;
         if (row < rows && tok < T) {
             const float *cv = ch[r][t];
             float a8[8];
@@ -515,11 +515,20 @@ hipError_t launch_router_batched(const DevTensor &R, const float *X, int T, cons
     const TopkArgs none{nullptr, 0, 0, nullptr, nullptr, nullptr};
     const int rows = (int)R.total_rows;
     *x_done = false;
-    if (R.type == 0 && R.cols % RT_KC == 0) {
-        const int gx = (rows + RT_RB - 1) / RT_RB;
-        *x_done = Xh && 4 * gx >= RT_TB;  // every token of a tile has a wavefront to convert it
-        hipLaunchKernelGGL(k_router_f32_tile, dim3(gx, (T + RT_TB - 1) / RT_TB), dim3(256), 0, s,
-                           (const float *)R.p0, X, bias, logits, rows, (int)R.cols, T, *x_done ? Xh : nullptr, rs);
+    if (R.type == 0 && R.cols % 256 == 0) {
+        auto tiles = [&](auto kernel, int RB, int TB) {
+            const int gx = (rows + RB - 1) / RB;
+            *x_done = Xh && 4 * gx >= TB;  // every token of a tile has a wavefront to convert it
+            hipLaunchKernelGGL(kernel, dim3(gx, (T + TB - 1) / TB), dim3(256), 0, s, (const float *)R.p0, X, bias,
+                               logits, rows, (int)R.cols, T, *x_done ? Xh : nullptr, rs);
+        };
+        // small tiles where the large ones are at most one block a CU (whole
+        // prefill calls, 128 rows, small | large: 37 tokens 65.5 | 70.4 us, 128
+        // 123.7 | 127.3, 200 104.1 | 104.5, 512 152.7 | 147.7)
+        if ((rows + 7) / 8 * ((T + 15) / 16) > 256)
+            tiles(k_router_f32_tile<8, 16, 128, 2>, 8, 16);
+        else
+            tiles(k_router_f32_tile<4, 8, 256, 4>, 4, 8);
     } else if (R.type == 0)
         hipLaunchKernelGGL(k_router_f32<64>, dim3((rows + 1) / 2, T), dim3(64), 0, s, (const float *)R.p0, X, bias,
                            logits, rows, (int)R.cols, none);

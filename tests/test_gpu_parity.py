@@ -1015,6 +1015,27 @@ def test_gpu_prefill_many_placement_tables(ctx, pool, T, E, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("T,E,D", [(1, 3, 256), (9, 65, 2304), (17, 130, 512),    # 4 x 8 tiles, 1, 9 and 2 stages
+                                   (515, 65, 768), (4100, 5, 256)])                # 8 x 16 tiles
+def test_gpu_prefill_router_tiles(ctx, T, E, D):
+    # the batched router's tiles, with ragged rows and tokens: selections and
+    # weights carry the bits of the one-token router
+    w = synth.moe_weights(91, D, E, 64, down_cols=256)
+    router, gate_up, down = lt.upload_moe(ctx, w)
+    X = synth.normal(synth.stream(92, T), (T, D))
+    k = min(E, 4)
+    out, ids, wt = np.zeros((T, D), np.float32), np.zeros((T, k), np.uint32), np.zeros((T, k), np.float32)
+    ctx.moe_prefill(out, X, router, gate_up, down, k, 64, norm_topk=True, out_ids=ids, out_w=wt)
+    one, w1 = np.zeros(k, np.uint32), np.zeros(k, np.float32)
+    for t in np.unique(np.r_[0, T - 1, np.arange(0, T, max(1, T // 40))]):
+        ctx.router_topk(router, X[t], k, one, w1, norm_topk=True)
+        assert np.array_equal(ids[t], one), t
+        assert np.array_equal(wt[t].view(np.uint32), w1.view(np.uint32)), t
+    for t in (router, gate_up, down):
+        t.free()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,E,k", [(1, 1, 1), (513, 3, 1), (1024, 128, 8), (8193, 5, 1), (70, 1024, 16)])
 def test_gpu_prefill_dispatch_edges(ctx, pool, T, E, k):
     # the placement, a block per expert: one assignment, a wavefront's share
