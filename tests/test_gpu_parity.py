@@ -992,6 +992,32 @@ def test_gpu_prefill_large_batches(ctx, pool, T, E, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("rows,cols", [
+    (1, 32), (5, 96),                    # less than 16 bytes out, and a last word that is not whole
+    (16384, 64), (16385, 64),            # the most that goes through pinned memory, and one row more
+    (300, 16384)])                       # the longest row in
+def test_gpu_host_vectors_match_device(ctx, rows, cols):
+    # host buffers of any address and length against device arrays: the same
+    # bits, nothing written past the end, and every call its own inputs
+    g = np.random.default_rng(rows + cols)
+    W = ctx.upload(synth.quant_matrix(g, ggml.Q8_0, rows, cols), ggml.Q8_0, rows, cols)
+    yd = hip.DeviceArray((rows,))
+    for call in range(6):
+        x = np.zeros(cols + 1, np.float32)[1:]
+        x[:] = g.standard_normal(cols)
+        out = np.full(rows + 9, 7.0, np.float32)
+        ctx.quant_matvec(out[1:rows + 1], W, x)
+        xd = hip.DeviceArray.from_numpy(np.ascontiguousarray(x))
+        ctx.quant_matvec(yd, W, xd)
+        ctx.sync()
+        assert np.array_equal(out[1:rows + 1].view(np.uint32), yd.numpy().view(np.uint32)), call
+        assert out[0] == 7.0 and (out[rows + 1:] == 7.0).all()
+        xd.free()
+    yd.free()
+    W.free()
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("T,E,k", [
     (3000, 128, 8),   # 24,000 assignments: three tables of eight rounds
     (2100, 256, 8),   # five tables of four rounds
