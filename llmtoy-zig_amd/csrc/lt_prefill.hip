@@ -394,8 +394,14 @@ __global__ void __launch_bounds__(512) k_prefill_dispatch(const uint32_t *__rest
     }
     const int tot_full = full >> 16, tot_two = two >> 16, n = cnt[e], nf = n / MC, rem = n % MC;
     if (e == 0 && tid == 0) *n_chunks = tot_full + tot_two + (one >> 16);
+    // The list's places go round the 8 XCDs, so full chunk f of 8 q (the rest
+    // at its own place) stands q places on in its XCD's row: the chunks of
+    // one expert run beside each other on one XCD, whose L2 then holds the
+    // weights they share (512 tokens 133.4 -> 131.6 us a call, 1024 209.3 -> 206.1).
+    const int per = tot_full / 8;
+    auto full_at = [&](int f) { return f < 8 * per ? f % per * 8 + f / per : f; };
     for (int c = tid; c < nf + (rem ? 1 : 0); c += 512) {
-        const int at = c < nf      ? (full & 0xffff) + c
+        const int at = c < nf      ? full_at((full & 0xffff) + c)
                        : rem > 32 ? tot_full + (two & 0xffff)
                                   : tot_full + tot_two + (one & 0xffff);
         chunks[3 * at] = e;
