@@ -124,7 +124,8 @@ template <class F>
 hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t s) {
     RowsPlan p{};
     p.U = (int)W.cols / F::kElems;
-    if (p.U > 512 || W.total_rows >= (size_t)1 << 30) return hipErrorInvalidValue;
+    // row indices are ints, and a last round's go up to 2 ND cap passes (2^21 rows) past the end
+    if (p.U > 512 || W.total_rows > ((size_t)1 << 31) - (1 << 22)) return hipErrorInvalidValue;
     // The workgroup size that leaves the fewest lanes idle, the largest of
     // them: x is staged once per workgroup (Q4_K 4,096 x 11,008 on 512 threads
     // 11.6 us, on 256 14.9; Q8_0 7,001 x 2,816 7.6 and 8.2).  A short matrix
