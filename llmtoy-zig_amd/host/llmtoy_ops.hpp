@@ -30,8 +30,10 @@
 // becomes Error::Unsupported.  Header-only; link with -lllmtoy_hip.
 #pragma once
 
+#include <algorithm>
 #include <cstddef>
 #include <cstdint>
+#include <cstring>
 #include <map>
 #include <memory>
 #include <optional>
@@ -102,7 +104,8 @@ class GpuContext {
         if (rc != LT_OK) throw Exception(Error::Device, rc, "lt_init failed (no usable device)");
     }
     ~GpuContext() {
-        for (auto &kv : cache_) lt_tensor_free(ctx_, kv.second);
+        for (auto &kv : cache_) lt_tensor_free(ctx_, kv.second.t);
+        for (lt_tensor *t : retired_) lt_tensor_free(ctx_, t);
         lt_destroy(ctx_);
     }
     GpuContext(const GpuContext &) = delete;
@@ -122,12 +125,16 @@ class GpuContext {
     // freeing or rewriting a buffer that was passed in.
     const lt_tensor *tensor(const RawMatrix &m, size_t n_experts = 1) {
         const Key key{m.data, m.rows, m.cols, n_experts};
+        const size_t bytes = m.rows * rowBytes(m.type, m.cols), head = std::min<size_t>(bytes, 256);
         auto it = cache_.find(key);
-        if (it != cache_.end()) return it->second;
+        // a new buffer at the address of one freed without forget(): the first
+        // bytes tell (the old copy lives on, a session may hold it)
+        if (it != cache_.end() && it->second.head.size() == head && !std::memcmp(it->second.head.data(), m.data, head))
+            return it->second.t;
         lt_tensor *t = nullptr;
-        check(lt_tensor_upload(ctx_, m.data, m.rows * rowBytes(m.type, m.cols), (uint32_t)m.type, m.rows / n_experts,
-                               m.cols, n_experts, &t));
-        cache_[key] = t;
+        check(lt_tensor_upload(ctx_, m.data, bytes, (uint32_t)m.type, m.rows / n_experts, m.cols, n_experts, &t));
+        if (it != cache_.end()) retired_.push_back(it->second.t);
+        cache_[key] = Copy{t, std::vector<uint8_t>(m.data, m.data + head)};
         return t;
     }
 
@@ -135,7 +142,7 @@ class GpuContext {
     void forget(const void *data) {
         for (auto it = cache_.begin(); it != cache_.end();) {
             if (it->first.data == data) {
-                lt_tensor_free(ctx_, it->second);
+                lt_tensor_free(ctx_, it->second.t);
                 it = cache_.erase(it);
             } else {
                 ++it;
@@ -155,7 +162,12 @@ class GpuContext {
         }
     };
     lt_ctx *ctx_ = nullptr;
-    std::map<Key, lt_tensor *> cache_;
+    struct Copy {
+        lt_tensor *t;
+        std::vector<uint8_t> head;  // the host bytes it was made from, up to 256
+    };
+    std::map<Key, Copy> cache_;
+    std::vector<lt_tensor *> retired_;
 };
 
 // ops/math.zig:133-171: out[rows] = mat . vec (fp32 activations).  The
