@@ -1,6 +1,7 @@
 // lt_matvec.hip -- matvec over rows of any length with fp32 activations:
-// Q8_0, and Q4_K / Q6_K rows that the streaming kernels (lt_q4k.hip,
-// lt_q6k.hip: 1, 2, 4, 8 or 16 super-blocks) do not take.
+// Q8_0, and the Q4_K / Q6_K matrices that the streaming kernels (lt_q4k.hip,
+// lt_q6k.hip: rows of 1, 2, 4, 8 or 16 super-blocks, and enough of them) do
+// not take.
 //
 // A row is U work units (Q8_0: a 32-element block; K-quants: 64 elements, a
 // Q4_K sub-block pair or a quarter of a Q6_K super-block).  A thread keeps
@@ -129,12 +130,16 @@ hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t
     // The workgroup size that leaves the fewest lanes idle, the largest of
     // them: x is staged once per workgroup (Q4_K 4,096 x 11,008 on 512 threads
     // 11.6 us, on 256 14.9; Q8_0 7,001 x 2,816 7.6 and 8.2).  A short matrix
-    // takes smaller ones until about 96 have a pass each (Q4_K 1,000 x 1,536:
-    // 3.9 us on 512, 3.4 on 256).
+    // takes smaller ones until 160 have a pass each (Q6_K 4,096 x 512: 3.19 us,
+    // 3.84 with 96, 3.11 with 256; 6,000 x 512 3.30, 4.02, 3.56), but less
+    // willingly where x is more than the two quads a thread that go ahead of
+    // the weights (Q6_K 1,000 x 1,536: 3.37 us on 192 threads, 3.71 on 128; Q8_0
+    // 200 x 4,096: 3.36 on 256, 3.70 on 128).
     double best = 0;
     for (int nt = 512; nt >= 128 && nt >= p.U; nt -= 64) {
         const int rp = nt / p.U, npass = (int)((W.total_rows + rp - 1) / rp);
-        const double used = (double)(rp * p.U) / nt * (npass >= 96 ? 1.0 : npass / 96.0);
+        const double used = (double)(rp * p.U) / nt * (npass >= 160 ? 1.0 : npass / 160.0) *
+                            (W.cols <= (size_t)8 * nt ? 1.0 : W.cols <= (size_t)16 * nt ? 0.75 : 0.4);
         if (used > best * 1.01) {
             best = used;
             p.nthreads = nt;

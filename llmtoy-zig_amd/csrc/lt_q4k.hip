@@ -204,7 +204,12 @@ static hipError_t launch_q4k_stream(const DevTensor &W, const float *x, float *y
 }
 
 hipError_t launch_matvec_q4k(const DevTensor &W, const float *x, float *y, hipStream_t s) {
-    if (W.total_rows * W.blocks_per_row < (size_t)1 << 31) {  // int row indices in the streaming kernel
+    // Small matrices are launch and round trip, and the conversion of x to
+    // limbs adds to them: streaming | rows, us, 1,000 x 512 3.77 | 2.79, 2,000 x
+    // 1,024 3.85 | 2.98, 4,096 x 1,024 3.98 | 3.76; 8,192 x 1,024 4.14 | 4.24,
+    // 4,096 x 4,096 4.46 | 5.43.  (At most int row indices in the streaming kernel.)
+    const size_t nsb = W.total_rows * W.blocks_per_row;
+    if (nsb > 16384 && nsb < (size_t)1 << 31) {
         switch (W.blocks_per_row) {
         case 1: return launch_q4k_stream<1>(W, x, y, s);
         case 2: return launch_q4k_stream<2>(W, x, y, s);

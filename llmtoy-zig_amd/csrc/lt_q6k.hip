@@ -170,6 +170,14 @@ static hipError_t launch_q6_stream(const DevTensor &W, const float *x, float *y,
 }
 
 hipError_t launch_matvec_q6k(const DevTensor &W, const float *x, float *y, hipStream_t s) {
+    // Small matrices: as in lt_q4k.hip (streaming | rows, us: 1,000 x 512 3.28 |
+    // 2.88, 6,000 x 512 3.88 | 3.30, 8,192 x 512 3.90 | 4.00; 2,000 x 1,024 3.85 |
+    // 3.19, 8,192 x 1,024 4.74 | 4.46, 12,000 x 1,024 5.34 | 5.39; 200 x 4,096
+    // 3.73 | 4.11, 2,000 x 4,096 4.93 | 4.60, 100,000 x 4,096 63.4 | 71.6: those
+    // stay streamed).
+    const size_t nsb = W.blocks_per_row;
+    if (nsb <= 8 && W.total_rows * nsb <= (nsb <= 2 ? 12288 : 32768))
+        return launch_matvec_rows(W, x, y, s);
     switch (W.blocks_per_row) {
     case 1: return launch_q6_stream<1>(W, x, y, s);
     case 2: return launch_q6_stream<2>(W, x, y, s);

@@ -292,7 +292,12 @@ def test_gpu_matvec_limb_nan(ctx, gtype, cols):
     (ggml.Q8_0, 30000, 96),
     (ggml.Q4_K, 3, 768), (ggml.Q4_K, 1001, 2816), (ggml.Q4_K, 37, 16384), (ggml.Q4_K, 30000, 768),
     (ggml.Q4_K, 300, 8192),                          # 32 super-blocks: 128 units
-    (ggml.Q6_K, 1, 768), (ggml.Q6_K, 999, 2816), (ggml.Q6_K, 37, 16384), (ggml.Q6_K, 30000, 768)])
+    (ggml.Q6_K, 1, 768), (ggml.Q6_K, 999, 2816), (ggml.Q6_K, 37, 16384), (ggml.Q6_K, 30000, 768),
+    # rows of a power of two of super-blocks: the largest that are not
+    # streamed, and fewer rows than a pass
+    (ggml.Q4_K, 1, 256), (ggml.Q4_K, 16384, 256), (ggml.Q4_K, 1024, 4096), (ggml.Q4_K, 333, 2048),
+    (ggml.Q6_K, 1, 256), (ggml.Q6_K, 12288, 256), (ggml.Q6_K, 6144, 512), (ggml.Q6_K, 8192, 1024),
+    (ggml.Q6_K, 4096, 2048), (ggml.Q6_K, 333, 2048)])
 def test_gpu_matvec_any_row_length(ctx, pool, gtype, rows, cols):
     # fp32 throughout: both sides round each of cols products and adds to
     # 2^-24 in chains of at most cols / 32 terms (the oracle's), so their
