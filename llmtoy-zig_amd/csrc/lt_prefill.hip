@@ -682,7 +682,7 @@ __device__ __forceinline__ uint32_t gate_up_tiles(const PfArgs &a, GemmLds &L, c
                                                   int mc, int col, int wave, int tid, int lane) {
     floatx16 acc[MT];
     uint32_t aoff[MT];
-    const float rt = a.rs[prow[min(tid, mc - 1)]];  // (rows past the chunk: its last row's)
+    const float rt = a.rs[prow[tid < mc ? tid : 0]];  // (rows past the chunk repeat its first one)
 #pragma unroll
     for (int t = 0; t < MT; t++) {
         const int m = 32 * t + (tid >> 3);
@@ -717,7 +717,9 @@ __device__ __forceinline__ uint32_t gate_up_tiles(const PfArgs &a, GemmLds &L, c
         top = fmaxf(top, fabsf(h));
         ht[BN1 * m] = (_Float16)h;
     });
-    if (top > 65504.0f)  // (rare: rows in range and finite values saturate and count, inf and NaN stay)
+    // (rare: rows in range and finite values saturate and count, inf and NaN
+    // stay; the whole wavefront goes, as each element needs its partner lane's half)
+    if (__any(top > 65504.0f))
         tile([&](int m, float h) {
             const bool big = fabsf(h) > 65504.0f && fabsf(h) <= 3.4e38f;
             sat += big && m < mc ? 1u : 0u;

@@ -959,6 +959,65 @@ def test_gpu_prefill_saturation_reported(ctx, pool):
         t.free()
 
 
+@pytest.mark.parametrize("act", [lt.ACT_SILU, lt.ACT_GELU_TANH])
+@pytest.mark.parametrize("T,at", [(9, 4), (9, 5), (40, 0), (40, 39), (70, 33), (70, 68)])
+def test_gpu_prefill_inf_row_harms_itself_only(ctx, T, at, act):
+    # one token's X holds an infinity and shares both experts with all the
+    # others (even and odd rows of one and two 32-row tiles, and of the short
+    # last chunk): the others carry the bits they have without it
+    w = synth.moe_weights(46, 256, 2, 64, down_cols=256)
+    X = synth.normal(synth.stream(46, T), (T, 256))
+    router, gate_up, down = lt.upload_moe(ctx, w)
+    clean, out = np.zeros((T, 256), np.float32), np.zeros((T, 256), np.float32)
+    ctx.moe_prefill(clean, X, router, gate_up, down, 2, 64, act=act)
+    X[at, 100] = np.inf
+    ctx.moe_prefill(out, X, router, gate_up, down, 2, 64, act=act)
+    others = np.arange(T) != at
+    assert np.array_equal(out[others].view(np.uint32), clean[others].view(np.uint32))
+    assert not np.isfinite(out[at]).any()
+    for t in (router, gate_up, down):
+        t.free()
+
+
+@pytest.mark.parametrize("T", [9, 40, 72])
+def test_gpu_prefill_one_column_saturates(ctx, T):
+    # one column of one expert overflows f16 for some of the tokens: the call
+    # counts exactly those activations and saturates them, and everything
+    # else is as without (f32 reference from dequantised weights; no
+    # activation within 5% of the limit, where f16 products could decide)
+    D, F, e, col = 256, 64, 1, 21
+    w = synth.moe_weights(47, D, 2, F, down_cols=256)
+    gu = w.gate_up.reshape(2, 2, F, 1, 144).copy()
+    gu[e, :, col, :, 0:2] = np.frombuffer(np.float16(0.2).tobytes(), np.uint8)
+    gu[e, :, col, :, 2:4] = np.frombuffer(np.float16(1.5).tobytes(), np.uint8)
+    w = dataclasses.replace(w, gate_up=gu.reshape(w.gate_up.shape))
+    X = synth.normal(synth.stream(47, T), (T, D))
+    gate_up = orc.dequant(orc.Q4_K, w.gate_up, w.gate_up.shape[0] * D).reshape(2, 2, F, D).astype(np.float64)
+    down = orc.dequant(orc.Q4_K, w.down, w.down.shape[0] * 256).reshape(2, D, 256).astype(np.float64)
+    X64 = X.astype(np.float64)
+    r2 = 4.0 ** np.floor(np.log2(np.abs(X64).max(axis=1, keepdims=True)))
+
+    def act(g):
+        return g / (1 + np.exp(-g))
+
+    with np.errstate(over="ignore"):
+        H = [act(X64 @ gate_up[q, 0].T) * (X64 @ gate_up[q, 1].T) / r2 for q in range(2)]
+    over = np.abs(H[e]) > 65504
+    assert over[:, col].any() and not over[:, col].all() and over.sum() == over[:, col].sum()
+    assert not (np.abs(H[0]) > 65504).any() and (np.abs(np.abs(H[e]) / 65504 - 1) > 0.05).all()
+    p = np.exp(X64 @ w.router.astype(np.float64).T)
+    p /= p.sum(axis=1, keepdims=True)
+    ref = sum(p[:, q:q + 1] * r2 * (np.clip(H[q], -65504, 65504) @ down[q, :, :F].T) for q in range(2))
+    t3 = lt.upload_moe(ctx, w)
+    out = np.zeros((T, D), np.float32)
+    with pytest.raises(DeviceError, match=f"prefill: {over.sum()} expert activations"):
+        ctx.moe_prefill(out, X, *t3, 2, F)
+    err = np.linalg.norm(out - ref, axis=1) / np.linalg.norm(ref, axis=1)
+    assert err.max() <= 2 * PREFILL_REL_L2, (int(err.argmax()), float(err.max()))  # (single rows)
+    for t in t3:
+        t.free()
+
+
 def test_gpu_prefill_deterministic(ctx, cfg3):
     c, (router, gate_up, down) = cfg3
     w = c["weights"]
