@@ -515,7 +515,7 @@ int matvec_dev(lt_ctx *ctx, const DevTensor &W, const float *x, float *y) {
     hipError_t e;
     switch (W.type) {
     case LT_TYPE_Q4_K: e = lt::launch_matvec_q4k(W, x, y, ctx->stream); break;
-    case LT_TYPE_Q8_0: e = lt::launch_matvec_rows(W, x, y, ctx->stream); break;
+    case LT_TYPE_Q8_0: e = lt::launch_matvec_q8_0(W, x, y, ctx->stream); break;
     case LT_TYPE_Q6_K: e = lt::launch_matvec_q6k(W, x, y, ctx->stream); break;
     case LT_TYPE_F32: e = lt::launch_matvec_f32(W, x, y, ctx->stream); break;
     case LT_TYPE_Q5_0:

@@ -374,6 +374,7 @@ hipError_t launch_matvec_q4k(const DevTensor &W, const float *x, float *y, hipSt
 // Q8_0, and Q4_K / Q6_K rows of any length (lt_matvec.hip); the launchers
 // above and below take the K-quant rows they stream themselves.
 hipError_t launch_matvec_rows(const DevTensor &W, const float *x, float *y, hipStream_t s);
+hipError_t launch_matvec_q8_0(const DevTensor &W, const float *x, float *y, hipStream_t s);
 hipError_t launch_matvec_q6k(const DevTensor &W, const float *x, float *y, hipStream_t s);
 hipError_t launch_matvec_f32(const DevTensor &W, const float *x, float *y, hipStream_t s);
 // Q5_0, Q5_1, IQ4_NL, Q3_K (lt_formats.hip)

@@ -148,6 +148,18 @@ static hipError_t launch_q8_any(const DevTensor &A, const DevTensor *B, const fl
     }
 }
 
+hipError_t launch_matvec_q8_0(const DevTensor &W, const float *x, float *y, hipStream_t s) {
+    // Small matrices, where each CU has little more than one workgroup: here |
+    // lt_matvec.hip, us, 1,000 x 256 2.33 | 2.39, 1,000 x 768 2.46 | 2.76, 2,500 x 512
+    // 2.50 | 2.68, 2,048 x 640 2.66 | 2.79, 600 x 1,536 2.73 | 2.85, 300 x 2,816 3.04 |
+    // 3.22; 4,096 x 256 2.79 | 2.48, 1,536 x 1,024 3.02 | 2.68, 512 x 2,560 3.51 | 3.17,
+    // 1,000 x 32 2.36 | 2.28.  Rows of 64 half blocks or less share wavefronts.
+    const size_t nu = W.blocks_per_row * 2, lanes = nu <= 64 ? nu : (nu + 63) / 64 * 64;
+    const size_t most = nu <= 16 || nu > 128 ? 61440 : 81920;
+    if (nu > 2 && nu <= 192 && W.total_rows * lanes <= most) return launch_q8_any<false>(W, nullptr, x, y, 0, s);
+    return launch_matvec_rows(W, x, y, s);
+}
+
 hipError_t launch_gate_up_q8_0(const DevTensor &Wg, const DevTensor &Wu, const float *x, uint32_t act, float *h,
                                hipStream_t s) {
     return launch_q8_any<true>(Wg, &Wu, x, h, act, s);

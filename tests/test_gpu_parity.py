@@ -311,6 +311,21 @@ def test_gpu_matvec_any_row_length(ctx, pool, gtype, rows, cols):
     assert rel_l2(y, ref) <= 3e-6, rel_l2(y, ref)
 
 
+@pytest.mark.parametrize("gtype,rows,cols", [
+    # Q8_0: the largest small matrix of each bound and one row more
+    (ggml.Q8_0, 3840, 256), (ggml.Q8_0, 3841, 256), (ggml.Q8_0, 2560, 512), (ggml.Q8_0, 2561, 512),
+    (ggml.Q8_0, 640, 2048), (ggml.Q8_0, 641, 2048), (ggml.Q8_0, 320, 3072), (ggml.Q8_0, 321, 3072), (ggml.Q8_0, 9, 32)])
+def test_gpu_matvec_launch_shapes(ctx, pool, gtype, rows, cols):
+    # (the bound of test_gpu_matvec_any_row_length)
+    g = np.random.default_rng(rows + cols)
+    w = synth.quant_matrix(g, gtype, rows, cols)
+    x = g.standard_normal(cols).astype(np.float32)
+    print(f"launch shape {ggml.NAMES[gtype]} {rows}x{cols}", flush=True)
+    y = gpu_matvec(ctx, w, gtype, rows, cols, x)
+    ref = orc.quant_matvec(w, gtype, x, rows, cols, pool=pool)
+    assert rel_l2(y, ref) <= 3e-6, rel_l2(y, ref)
+
+
 @pytest.mark.parametrize("gtype,cols", [(ggml.Q8_0, 2080), (ggml.Q8_0, 256), (ggml.Q4_K, 768), (ggml.Q6_K, 768)])
 def test_gpu_matvec_any_row_length_nan_inf_small(ctx, gtype, cols):
     # NaN reaches every output; an infinity gives what the oracle gives;
