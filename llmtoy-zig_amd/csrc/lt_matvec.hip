@@ -14,9 +14,9 @@
 // What bounds it: HBM on large matrices, the launch and a round trip to
 // memory on small ones.  Measured (us a launch, cold weights, the kernels
 // this replaces -> here): Q6_K 262,144 x 2,816 188 -> 115 (5.3 TB/s), 4,096 x
-// 2,816 7.9 -> 5.8; Q4_K 40,000 x 2,560 23.1 -> 17.7, 4,096 x 2,816 7.5 ->
-// 5.2, 2,048 x 5,120 10.4 -> 5.5; Q8_0 7,001 x 2,816 9.3 -> 7.6, 4,096 x
-// 4,096 10.2 -> 6.4, 151,936 x 896 31.0 -> 26.8, 600 x 512 2.3 -> 2.4.  The
+// 2,816 6.9 -> 5.5; Q4_K 40,000 x 2,560 21.0 -> 16.7, 4,096 x 2,816 6.6 ->
+// 4.9, 2,816 x 5,120 9.1 -> 5.9; Q8_0 7,001 x 2,816 8.0 -> 6.9, 4,096 x
+// 4,096 9.0 -> 6.0, 152,000 x 2,048 62 -> 62, 152,000 x 896 33 -> 27.  The
 // old kernels put a power of two of lanes on a row (11 super-blocks: a third
 // of them idle), waited for x before they requested a weight, and converted
 // every code.  Activations as three int8 limbs against v_dot4 instead were
@@ -31,9 +31,9 @@ namespace lt {
 namespace {
 
 // A pass is RP rows of U units on nthreads = blockDim threads; T = 2^logT
-// threads add up a row.
+// threads add up a row; nd load buffers.
 struct RowsPlan {
-    int U, RP, nthreads, nblk, logT, npass;
+    int U, RP, nthreads, nblk, logT, npass, nd;
 };
 
 }  // namespace
@@ -121,12 +121,52 @@ hipError_t launch_rows_t(const DevTensor &W, const float *x, float *y, RowsPlan 
     return hipGetLastError();
 }
 
+// A launch of nt threads a workgroup and nd load buffers, on up to waves
+// wavefronts a CU.
+RowsPlan rows_plan(const DevTensor &W, int U, int nt, int nd, int waves) {
+    RowsPlan p{};
+    p.U = U;
+    p.nthreads = nt;
+    p.RP = nt / U;
+    p.npass = (int)((W.total_rows + p.RP - 1) / p.RP);
+    p.nblk = std::min(p.npass, 256 * (waves * 64 / nt));
+    p.nd = nd;
+    return p;
+}
+
+// An estimate of the launch, as bytes that the CU with the most passes reads:
+// its weights, with passes in rounds of nd (F::kRound of the time, as more is
+// in flight), times (F::kLanes / lanes)^3 where the matrix fills the chip and
+// the lanes at work on a CU are fewer than that; twice the x that its
+// workgroups stage; and 3,000 for every round of x loads behind the two quads
+// a thread that go ahead of the weights.  Fitted to 570 sizes: the shape of
+// the least estimate takes 1.03 of the best shape's time on the average.
+template <class F>
+double rows_cost(const DevTensor &W, RowsPlan p) {
+    const int lds = (int)W.cols * 4 + p.nd * 4096;  // of a workgroup
+    p.nblk = std::min(p.nblk, 256 * ((160 << 10) / lds));
+    int passes = 0;
+    for (int b = 0; b < p.nblk; b += 256) {
+        const int n = (p.npass - b + p.nblk - 1) / p.nblk;
+        passes += (n + p.nd - 1) / p.nd * p.nd;
+    }
+    double t = (double)p.RP * passes * (W.bytes / W.total_rows) * (p.nd > 1 ? F::kRound : 1.0);
+    if (p.npass > p.nblk) {
+        const double few = std::max(1.0, F::kLanes / (p.nblk / 256 * p.RP * p.U));
+        t *= few * few * few;
+    }
+    const int late = std::max(0, ((int)W.cols / 4 - 2 * p.nthreads + p.nthreads - 1) / p.nthreads);
+    return t + 2.0 * ((p.nblk + 255) / 256) * W.cols * 4 + 3000.0 * late;
+}
+
 template <class F>
 hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t s) {
-    RowsPlan p{};
-    p.U = (int)W.cols / F::kElems;
+    const int U = (int)W.cols / F::kElems;
     // row indices are ints, and a last round's go up to 2 ND cap passes (2^21 rows) past the end
-    if (p.U > 512 || W.total_rows > ((size_t)1 << 31) - (1 << 22)) return hipErrorInvalidValue;
+    if (U > 512 || W.total_rows > ((size_t)1 << 31) - (1 << 22)) return hipErrorInvalidValue;
+    // up to two passes a workgroup: one load buffer, as the others would load
+    // rows again that nobody needs (Q8_0 4,096 x 4,096: 6.3 us, 7.1 with four)
+    auto runs = [&](int nt) { return rows_plan(W, U, nt, 1, 16).npass > 2 * 256 * (1024 / nt); };
     // The workgroup size that leaves the fewest lanes idle, the largest of
     // them: x is staged once per workgroup (Q4_K 4,096 x 11,008 on 512 threads
     // 11.6 us, on 256 14.9; Q8_0 7,001 x 2,816 7.6 and 8.2).  A short matrix
@@ -136,25 +176,41 @@ hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t
     // the weights (Q6_K 1,000 x 1,536: 3.37 us on 192 threads, 3.71 on 128; Q8_0
     // 200 x 4,096: 3.36 on 256, 3.70 on 128).
     double best = 0;
-    for (int nt = 512; nt >= 128 && nt >= p.U; nt -= 64) {
-        const int rp = nt / p.U, npass = (int)((W.total_rows + rp - 1) / rp);
-        const double used = (double)(rp * p.U) / nt * (npass >= 160 ? 1.0 : npass / 160.0) *
+    RowsPlan p{};
+    for (int nt = 512; nt >= 128 && nt >= U; nt -= 64) {
+        const RowsPlan q = rows_plan(W, U, nt, runs(nt) ? F::ND : 1, 16);
+        const double used = (double)(q.RP * U) / nt * (q.npass >= 160 ? 1.0 : q.npass / 160.0) *
                             (W.cols <= (size_t)8 * nt ? 1.0 : W.cols <= (size_t)16 * nt ? 0.75 : 0.4);
         if (used > best * 1.01) {
             best = used;
-            p.nthreads = nt;
+            p = q;
         }
     }
-    p.RP = p.nthreads / p.U;
-    p.npass = (int)((W.total_rows + p.RP - 1) / p.RP);
-    const int cap = 256 * (1024 / p.nthreads);  // resident workgroups: 16 wavefronts a CU
-    p.nblk = std::min(p.npass, cap);
-    // up to two passes a workgroup: one load buffer, as the others would load
-    // rows again that nobody needs (Q8_0 4,096 x 4,096: 6.3 us, 7.1 with four)
-    const bool one = p.npass <= 2 * cap;
-    if (p.U <= 64 && (p.U & (p.U - 1)) == 0)
-        return one ? launch_rows_t<F, 1, true>(W, x, y, p, s) : launch_rows_t<F, F::ND, true>(W, x, y, p, s);
-    return one ? launch_rows_t<F, 1, false>(W, x, y, p, s) : launch_rows_t<F, F::ND, false>(W, x, y, p, s);
+    // That shape does not see passes that go unevenly over the CUs, or come in
+    // whole rounds: another one whose estimate is clearly less (F::kKeep) takes
+    // its place, but for K-quants not in long runs, where unevenness is small and
+    // the estimate errs by as much (Q6_K 262,144 x 2,816: 114 us kept, 131
+    // replaced).  Kept | replaced, us: Q6_K 7,001 x 5,120 15.9 | 10.1; Q4_K 16,000 x
+    // 1,280 7.2 | 5.7, 7,001 x 5,120 12.4 | 8.6; Q8_0 152,000 x 512 19.4 | 16.1,
+    // 11,000 x 2,048 8.5 | 6.8, 2,816 x 4,864 7.2 | 6.4; the other way Q4_K 16,000 x
+    // 1,792 6.6 | 7.1, Q6_K 11,000 x 1,536 6.3 | 6.6.
+    if (p.npass <= F::kLong * p.nblk) {
+        double least =
+            F::kKeep * rows_cost<F>(W, rows_plan(W, U, p.nthreads, p.nd, p.nd == 1 ? F::waves(U) : 16));
+        for (int nt = 512; nt >= 128 && nt >= U; nt -= 64)
+            for (int nd : {1, F::ND}) {
+                if (!F::takes(U, nd, runs(nt))) continue;
+                const RowsPlan q = rows_plan(W, U, nt, nd, nd == 1 ? F::waves(U) : 16);
+                const double cost = rows_cost<F>(W, q);
+                if (cost < least) {
+                    least = cost;
+                    p = q;
+                }
+            }
+    }
+    if (U <= 64 && (U & (U - 1)) == 0)
+        return p.nd == 1 ? launch_rows_t<F, 1, true>(W, x, y, p, s) : launch_rows_t<F, F::ND, true>(W, x, y, p, s);
+    return p.nd == 1 ? launch_rows_t<F, 1, false>(W, x, y, p, s) : launch_rows_t<F, F::ND, false>(W, x, y, p, s);
 }
 
 }  // namespace

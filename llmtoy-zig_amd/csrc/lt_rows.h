@@ -37,9 +37,17 @@ __device__ __forceinline__ float sum16(const float *v) {
 
 // ---- formats: elements per unit (kElems), the unit and quad within it of
 // activations 4 f + [0, 4), the unit's activations from its quads, the loads
-// of unit i behind unit u0 of the matrix, and the unit's dot product.
+// of unit i behind unit u0 of the matrix, and the unit's dot product.  For the
+// matvec's launch shapes (lt_matvec.hip): load buffers in runs of many passes
+// (ND), the wavefronts that a CU holds with one buffer (waves: the registers
+// allow 32 for Q8_0, but rows of more than 256 units take as much LDS for x
+// that fewer are better), the numbers of buffers to choose from (takes), and
+// the constants of its estimate.
 struct FmtQ8_0 {
     static constexpr int kElems = 32, ND = 4;
+    static constexpr double kRound = 0.85, kLanes = 1536, kKeep = 0.85, kLong = 1e9;
+    static int waves(int U) { return U <= 256 ? 32 : 16; }
+    static bool takes(int U, int nd, bool runs) { return (nd > 1) == (runs && U > 256); }
     struct X {
         float v[32];
     };
@@ -72,6 +80,9 @@ struct FmtQ8_0 {
 
 struct FmtQ4_K {
     static constexpr int kElems = 64, ND = 2;
+    static constexpr double kRound = 0.9, kLanes = 1024, kKeep = 0.94, kLong = 6;
+    static int waves(int) { return 16; }
+    static bool takes(int, int nd, bool runs) { return nd == 1 || runs; }
     struct X {
         float v[64], s[4];  // the activations and the sums of their groups of 16
     };
@@ -116,6 +127,9 @@ struct FmtQ4_K {
 
 struct FmtQ6_K {
     static constexpr int kElems = 64, ND = 2;
+    static constexpr double kRound = 1.0, kLanes = 1024, kKeep = 0.94, kLong = 6;
+    static int waves(int) { return 16; }
+    static bool takes(int, int nd, bool runs) { return nd == 1 || runs; }
     struct X {
         float v[64], s[4];  // four groups of 16, and -32 times their sums
     };

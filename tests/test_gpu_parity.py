@@ -314,7 +314,12 @@ def test_gpu_matvec_any_row_length(ctx, pool, gtype, rows, cols):
 @pytest.mark.parametrize("gtype,rows,cols", [
     # Q8_0: the largest small matrix of each bound and one row more
     (ggml.Q8_0, 3840, 256), (ggml.Q8_0, 3841, 256), (ggml.Q8_0, 2560, 512), (ggml.Q8_0, 2561, 512),
-    (ggml.Q8_0, 640, 2048), (ggml.Q8_0, 641, 2048), (ggml.Q8_0, 320, 3072), (ggml.Q8_0, 321, 3072), (ggml.Q8_0, 9, 32)])
+    (ggml.Q8_0, 640, 2048), (ggml.Q8_0, 641, 2048), (ggml.Q8_0, 320, 3072), (ggml.Q8_0, 321, 3072), (ggml.Q8_0, 9, 32),
+    # one buffer in long runs, and four where a row is the most of a pass
+    (ggml.Q8_0, 40001, 2048), (ggml.Q8_0, 16001, 4864), (ggml.Q8_0, 3001, 11008),
+    # K-quants: shapes taken for even passes, and a long run that keeps the first choice
+    (ggml.Q4_K, 16001, 1280), (ggml.Q4_K, 7001, 5120), (ggml.Q4_K, 40001, 1792), (ggml.Q6_K, 7001, 5120),
+    (ggml.Q6_K, 4099, 8448), (ggml.Q6_K, 30001, 1792)])
 def test_gpu_matvec_launch_shapes(ctx, pool, gtype, rows, cols):
     # (the bound of test_gpu_matvec_any_row_length)
     g = np.random.default_rng(rows + cols)
