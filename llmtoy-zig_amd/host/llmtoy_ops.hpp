@@ -31,6 +31,7 @@
 #pragma once
 
 #include <algorithm>
+#include <array>
 #include <cstddef>
 #include <cstdint>
 #include <cstring>
@@ -104,8 +105,8 @@ class GpuContext {
         if (rc != LT_OK) throw Exception(Error::Device, rc, "lt_init failed (no usable device)");
     }
     ~GpuContext() {
-        for (auto &kv : cache_) lt_tensor_free(ctx_, kv.second.t);
-        for (lt_tensor *t : retired_) lt_tensor_free(ctx_, t);
+        for (auto &kv : cache_)
+            for (const Copy &c : kv.second) lt_tensor_free(ctx_, c.t);
         lt_destroy(ctx_);
     }
     GpuContext(const GpuContext &) = delete;
@@ -118,23 +119,31 @@ class GpuContext {
     }
 
     // The device copy of m viewed as n_experts matrices of rows/n_experts
-    // rows (uploaded on first use, cached by data pointer and shape).  As in
-    // the reference (the GGUF mmap must outlive the weights,
+    // rows (uploaded on first use, cached by data pointer, type and shape).  As
+    // in the reference (the GGUF mmap must outlive the weights,
     // model/model_weights.zig:11), the host bytes must stay alive and
-    // unchanged while the context may use them; call forget() before
-    // freeing or rewriting a buffer that was passed in.
+    // unchanged while the context may use them; call forget() before freeing or
+    // rewriting a buffer that was passed in.  Where that was left out, 16 pieces
+    // of 64 bytes, spread over the matrix, tell another matrix at the same
+    // address; a change between them they do not see.  Each matrix that was seen
+    // at an address keeps its copy until forget(), as a session may hold it.
     const lt_tensor *tensor(const RawMatrix &m, size_t n_experts = 1) {
-        const Key key{m.data, m.rows, m.cols, n_experts};
-        const size_t bytes = m.rows * rowBytes(m.type, m.cols), head = std::min<size_t>(bytes, 256);
-        auto it = cache_.find(key);
-        // a new buffer at the address of one freed without forget(): the first
-        // bytes tell (the old copy lives on, a session may hold it)
-        if (it != cache_.end() && it->second.head.size() == head && !std::memcmp(it->second.head.data(), m.data, head))
-            return it->second.t;
-        lt_tensor *t = nullptr;
+        const size_t bytes = m.rows * rowBytes(m.type, m.cols);
+        const Key key{m.data, (uint32_t)m.type, m.rows, m.cols, n_experts};
+        const auto it = cache_.find(key);
+        if (it != cache_.end()) {
+            const Mark now = mark(m.data, bytes);
+            for (const Copy &c : it->second)
+                if (c.mark == now) return c.t;
+        }
+        lt_tensor *t = nullptr;  // (before its bytes are read here: refuses what cannot be uploaded)
         check(lt_tensor_upload(ctx_, m.data, bytes, (uint32_t)m.type, m.rows / n_experts, m.cols, n_experts, &t));
-        if (it != cache_.end()) retired_.push_back(it->second.t);
-        cache_[key] = Copy{t, std::vector<uint8_t>(m.data, m.data + head)};
+        try {
+            cache_[key].push_back(Copy{t, mark(m.data, bytes)});
+        } catch (...) {
+            lt_tensor_free(ctx_, t);
+            throw;
+        }
         return t;
     }
 
@@ -142,7 +151,7 @@ class GpuContext {
     void forget(const void *data) {
         for (auto it = cache_.begin(); it != cache_.end();) {
             if (it->first.data == data) {
-                lt_tensor_free(ctx_, it->second.t);
+                for (const Copy &c : it->second) lt_tensor_free(ctx_, c.t);
                 it = cache_.erase(it);
             } else {
                 ++it;
@@ -150,24 +159,42 @@ class GpuContext {
         }
     }
 
+    // Device copies held.
+    size_t copies() const {
+        size_t n = 0;
+        for (const auto &kv : cache_) n += kv.second.size();
+        return n;
+    }
+
    private:
     struct Key {
         const uint8_t *data;
+        uint32_t type;
         size_t rows, cols, n_experts;
         bool operator<(const Key &o) const {
             if (data != o.data) return data < o.data;
+            if (type != o.type) return type < o.type;
             if (rows != o.rows) return rows < o.rows;
             if (cols != o.cols) return cols < o.cols;
             return n_experts < o.n_experts;
         }
     };
-    lt_ctx *ctx_ = nullptr;
+    static constexpr size_t kPieces = 16;
+    using Mark = std::array<uint8_t, kPieces * 64>;  // the host bytes compared
     struct Copy {
         lt_tensor *t;
-        std::vector<uint8_t> head;  // the host bytes it was made from, up to 256
+        Mark mark;
     };
-    std::map<Key, Copy> cache_;
-    std::vector<lt_tensor *> retired_;
+    static Mark mark(const uint8_t *data, size_t bytes) {
+        Mark r{};
+        const size_t piece = std::min(bytes, r.size() / kPieces);
+        for (size_t i = 0; i < kPieces; i++)  // (the last piece is the matrix's last)
+            std::memcpy(r.data() + i * piece,
+                        data + (i + 1 < kPieces ? (bytes - piece) / (kPieces - 1) * i : bytes - piece), piece);
+        return r;
+    }
+    lt_ctx *ctx_ = nullptr;
+    std::map<Key, std::vector<Copy>> cache_;  // by address: the matrices seen there
 };
 
 // ops/math.zig:133-171: out[rows] = mat . vec (fp32 activations).  The

@@ -1,6 +1,7 @@
 // Parity tests of the C++ host layer (llmtoy-zig_amd/host/llmtoy_ops.hpp)
 // against the CPU oracle, named after the reference's own test blocks.
-// Run with a GPU: ./test_host_ops ; without one: ./test_host_ops --list.
+// Run with a GPU: ./test_host_ops, ./test_host_ops --cache ; without one:
+// ./test_host_ops --list.
 #include <cmath>
 #include <cstdio>
 #include <cstring>
@@ -250,8 +251,61 @@ static void test_run_moe_block(GpuContext &g) {  // gemma4/forward.zig:403-497
     EXPECT(rel_l2(x, ref) < 1e-3);
 }
 
+// The context's device copies (--cache): what stands at the address of a
+// buffer that was rewritten or freed without forget(), and what forget() frees.
+static bool matches(GpuContext &g, const RawMatrix &m, const std::vector<float> &vec) {
+    std::vector<float> out(m.rows), ref(m.rows), rowbuf(m.cols);
+    quantMatvec(g, out.data(), m, vec.data());
+    lto_quant_matvec(ref.data(), m.data, (uint32_t)m.type, vec.data(), m.rows, m.cols, rowbuf.data());
+    return max_rel(out, ref) < 1e-4;
+}
+
+static void test_cache(GpuContext &g) {
+    const size_t rows = 64, cols = 2048, n = rows * rowBytes(GgmlType::q4_k, cols);
+    const auto a = fuzz_matrix(GgmlType::q4_k, rows, cols, 7), b = fuzz_matrix(GgmlType::q4_k, rows, cols, 8);
+    std::vector<float> vec(cols);
+    Rng r{9};
+    for (auto &v : vec) v = (r.uniform() - 0.5f) * 2.0f;
+    std::vector<uint8_t> buf(rows * rowBytes(GgmlType::q6_k, cols));
+    std::memcpy(buf.data(), a.data(), n);
+    const RawMatrix m{buf.data(), n, GgmlType::q4_k, rows, cols};
+    const size_t before = g.copies();
+    EXPECT(matches(g, m, vec));
+    const lt_tensor *ta = g.tensor(m);
+    // another matrix whose first rows are the same, then the two in turn: each
+    // has one copy, however often it comes back
+    std::memcpy(buf.data() + 8 * rowBytes(GgmlType::q4_k, cols), b.data(), n - 8 * rowBytes(GgmlType::q4_k, cols));
+    EXPECT(matches(g, m, vec));
+    const std::vector<uint8_t> ab(buf.begin(), buf.begin() + n);
+    for (int i = 0; i < 6; i++) {
+        std::memcpy(buf.data(), i & 1 ? ab.data() : a.data(), n);
+        EXPECT(matches(g, m, vec));
+        EXPECT((g.tensor(m) == ta) == !(i & 1));
+    }
+    EXPECT(g.copies() == before + 2);
+    // the same bytes as another type of the same rows and columns
+    const auto c = fuzz_matrix(GgmlType::q6_k, rows, cols, 10);
+    std::memcpy(buf.data(), c.data(), c.size());
+    EXPECT(matches(g, {buf.data(), c.size(), GgmlType::q6_k, rows, cols}, vec));
+    const auto e = fuzz_matrix(GgmlType::q4_k, rows, cols, 11);
+    std::memcpy(buf.data(), e.data(), n);
+    EXPECT(matches(g, {buf.data(), c.size(), GgmlType::q6_k, rows, cols}, vec));
+    EXPECT(matches(g, m, vec));
+    // forget() drops every copy made from the address; a change of one byte
+    // between the compared ones is seen behind it
+    g.forget(buf.data());
+    EXPECT(g.copies() == before);
+    EXPECT(matches(g, m, vec));
+    buf[n / 2 + 300] ^= 0xff;
+    g.forget(buf.data());
+    EXPECT(matches(g, m, vec));
+    g.forget(buf.data());
+    EXPECT(g.copies() == before);
+}
+
 int main(int argc, char **argv) {
-    const std::vector<std::pair<std::string, std::function<void(GpuContext &)>>> tests = {
+    const bool cache = argc > 1 && std::strcmp(argv[1], "--cache") == 0;
+    std::vector<std::pair<std::string, std::function<void(GpuContext &)>>> tests = {
         {"gpu matvec Q8_0 correctness", test_q8_0_correctness},
         {"gpu matvec Q4_K scale", test_q4_k_scale},
         {"gpu matvec Q4_K min", test_q4_k_min},
@@ -269,6 +323,7 @@ int main(int argc, char **argv) {
         for (auto &t : tests) std::printf("%s\n", t.first.c_str());
         return 0;
     }
+    if (cache) tests = {{"GpuContext: device copies of rewritten buffers", test_cache}};
     try {
         GpuContext g(0);
         for (auto &t : tests) {

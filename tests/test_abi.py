@@ -70,6 +70,15 @@ def test_gpu_cpp_host_layer_parity():
     assert out.returncode == 0 and "ALL PASSED" in out.stdout, out.stdout + out.stderr
 
 
+@pytest.mark.gpu
+def test_gpu_cpp_host_cache():
+    # device copies of host buffers that are rewritten, freed and forgotten
+    print("running tests/cpp/build/test_host_ops --cache", flush=True)
+    out = subprocess.run([CPP_TEST, "--cache"], capture_output=True, text=True, timeout=120)
+    print(out.stdout[-3000:])
+    assert out.returncode == 0 and "ALL PASSED" in out.stdout, out.stdout + out.stderr
+
+
 def test_null_arguments_are_invalid_without_touching_a_device():
     L = lt.load_library()
     assert L.lt_init(0, None) == ltlib.LT_ERR_INVALID
