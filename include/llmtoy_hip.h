@@ -141,12 +141,19 @@ int lt_stream_read(lt_ctx *ctx, const void *buf, size_t nbytes);
 size_t lt_tensor_bytes(const lt_tensor *t);
 
 /* out[rows] = W[rows x cols] * x[cols], fp32 accumulation.  Activations are
- * fp32, except for Q4_K and Q6_K rows of 1, 2, 4, 8 or 16 super-blocks
- * (cols 256..4096, powers of two): there each group of 16 activations is
- * split into two int8 limbs, x ~= sp * (256 a + b) with sp = max|x| / 32512
- * (|error| <= max|x| / 65024 per element, about 2e-5 rel-L2 on the dot
- * product), which meet the weight codes in v_dot4; a group holding a NaN or
- * an infinity makes every output NaN.
+ * fp32, except for large Q4_K and Q6_K matrices with rows of 1, 2, 4, 8 or 16
+ * super-blocks (cols 256..4096, powers of two): Q4_K of more than 16,384
+ * super-blocks in all, Q6_K of more than 12,288 (rows of 1 or 2) or 32,768
+ * (rows of 4 or 8) or of any number (rows of 16).  There each group of 16
+ * activations is split into two int8 limbs, x ~= sp * (256 a + b) with sp =
+ * max|x| / 32512 (|error| <= max|x| / 65024 per element, about 2e-5 rel-L2 on
+ * the dot product), which meet the weight codes in v_dot4; a group holding a
+ * NaN or an infinity makes every output NaN.  So the rounding, and what an
+ * infinity gives, depend on the number of rows: with fp32 activations a NaN
+ * makes every output NaN too, but an infinity gives what the products and
+ * sums give, which is NaN or an infinity (Q4_K and Q6_K subtract a block's
+ * offset as a sum of its own, Q8_0 has none).  Q4_K and Q6_K activations below
+ * about 2^-100 lose bits (their products are kept 2^-24 of their size).
  * Replaces quantMatvec / quantMatvecPar (ops/math.zig:133-171, 277-320) and
  * MatvecSession.run / runQ8_1Mv (gpu/matvec.zig:497-647,
  * gemma4/gpu_weights.zig:1573-1607).  W must be a 2-D tensor. */
@@ -234,7 +241,7 @@ int lt_moe_forward_noalloc(lt_ctx *ctx, float *out, const float *x, const lt_ten
 /* Batched prefill of one MoE layer over T tokens (X, out: [T, d_model]):
  * per-token routing as lt_moe_router_topk, tokens sorted per expert, grouped
  * expert GEMM with f16 MFMA (fp32 accumulation) over Q4_K weights
- * dequantised in LDS, then a combine in slot order.  The reference prefills
+ * dequantised in registers, then a combine in slot order.  The reference prefills
  * one token at a time through the decode path (main.zig:1916-1922); results
  * match per-token lt_moe_forward to f16 tolerance.  Each X row is divided by
  * a power of two 2^e that puts its largest element in [1, 2) and the expert
@@ -242,7 +249,9 @@ int lt_moe_forward_noalloc(lt_ctx *ctx, float *out, const float *x, const lt_ten
  * exact rescaling), so rows of any magnitude stay inside f16's range; an
  * activation that still passes +-65504 saturates there, is counted, and the
  * call (LT_HOST_IO) or the next lt_sync returns LT_ERR_DEVICE naming the
- * count.  Device pointers X and out must be 16-byte aligned. */
+ * count.  A NaN or an infinity in a row of X makes that row's output NaN or
+ * infinite and leaves the other rows as they are.  Device pointers X and out
+ * must be 16-byte aligned. */
 int lt_moe_prefill(lt_ctx *ctx, float *out, const float *X, uint32_t T, const lt_tensor *router,
                    const float *router_bias, const lt_tensor *gate_up, const lt_tensor *down, uint32_t k,
                    uint32_t d_expert, uint32_t act, uint32_t flags, uint32_t *out_ids, float *out_w);

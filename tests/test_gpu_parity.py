@@ -284,6 +284,32 @@ def test_gpu_matvec_limb_nan(ctx, gtype, cols):
     assert np.isnan(y).all()
 
 
+@pytest.mark.parametrize("gtype,rows,cols,limbs", [
+    (ggml.Q4_K, 16384, 256, False), (ggml.Q4_K, 16385, 256, True),
+    (ggml.Q4_K, 1024, 4096, False), (ggml.Q4_K, 1025, 4096, True),
+    (ggml.Q6_K, 12288, 256, False), (ggml.Q6_K, 12289, 256, True),
+    (ggml.Q6_K, 6144, 512, False), (ggml.Q6_K, 6145, 512, True),
+    (ggml.Q6_K, 8192, 1024, False), (ggml.Q6_K, 8193, 1024, True),
+    (ggml.Q6_K, 4096, 2048, False), (ggml.Q6_K, 4097, 2048, True), (ggml.Q6_K, 3, 4096, True)])
+def test_gpu_matvec_limb_bounds(ctx, pool, gtype, rows, cols, limbs):
+    # int8 limbs from a number of super-blocks on, fp32 activations below it:
+    # which one it is shows in the rounding (2e-5 of two limbs, 1e-7 of fp32);
+    # a NaN reaches every output of both, an infinity makes every output NaN
+    # with limbs, NaN or infinite without
+    g = np.random.default_rng(rows + cols)
+    w = synth.quant_matrix(g, gtype, rows, cols)
+    x = g.standard_normal(cols).astype(np.float32)
+    print(f"limb bounds {ggml.NAMES[gtype]} {rows}x{cols}", flush=True)
+    ref = orc.quant_matvec(w, gtype, x, rows, cols, pool=pool)
+    e = rel_l2(gpu_matvec(ctx, w, gtype, rows, cols, x), ref)
+    assert (5e-6 <= e <= 1e-4) if limbs else e <= 3e-6, e
+    x[cols // 3] = np.nan
+    assert np.isnan(gpu_matvec(ctx, w, gtype, rows, cols, x)).all()
+    x[cols // 3] = np.inf
+    y = gpu_matvec(ctx, w, gtype, rows, cols, x)
+    assert np.isnan(y).all() if limbs else not np.isfinite(y).any()
+
+
 @pytest.mark.parametrize("gtype,rows,cols", [
     (ggml.Q8_0, 1, 32), (ggml.Q8_0, 131, 64),        # rows of one and two units, inside a wavefront
     (ggml.Q8_0, 70, 2080), (ggml.Q8_0, 7001, 2816),  # 65 and 88 units: rows straddle wavefronts
