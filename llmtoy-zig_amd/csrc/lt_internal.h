@@ -181,48 +181,6 @@ __device__ __forceinline__ float wave_sum_transposed(float (&v)[V], int lane, bo
     return t;
 }
 
-// Sums V values (V = 1, 2, 4 or 8) over each aligned group of 8 lanes.
-// Returns, in lane g*8 + j, the group's total of value index j * V / 8
-// (for V = 8: value j).
-template <int V>
-__device__ __forceinline__ float group8_sum_transposed(float (&v)[V], int lane) {
-    static_assert(V == 1 || V == 2 || V == 4 || V == 8, "V");
-    float a[V];
-#pragma unroll
-    for (int i = 0; i < V; i++) a[i] = v[i];
-    int n = V;
-    if (n > 1) {  // lane bit 2: row_half_mirror pairs i with 7 - i
-        const bool hi = lane & 4;
-#pragma unroll
-        for (int i = 0; i < V / 2; i++) {
-            const float send = hi ? a[i] : a[i + V / 2], keep = hi ? a[i + V / 2] : a[i];
-            a[i] = keep + dpp<0x141>(send);
-        }
-        n = V / 2;
-    } else {
-        a[0] += dpp<0x141>(a[0]);
-    }
-    if (n > 1) {  // lane bit 1
-        const bool hi = lane & 2;
-#pragma unroll
-        for (int i = 0; i < V / 4; i++) {
-            const float send = hi ? a[i] : a[i + V / 4], keep = hi ? a[i + V / 4] : a[i];
-            a[i] = keep + dpp<0x4E>(send);
-        }
-        n = V / 4;
-    } else {
-        a[0] += dpp<0x4E>(a[0]);
-    }
-    if (n > 1) {  // lane bit 0
-        const bool hi = lane & 1;
-        const float send = hi ? a[0] : a[1], keep = hi ? a[1] : a[0];
-        a[0] = keep + dpp<0xB1>(send);
-    } else {
-        a[0] += dpp<0xB1>(a[0]);
-    }
-    return a[0];
-}
-
 __device__ __forceinline__ float act_silu(float g) { return g / (1.0f + __expf(-g)); }
 
 __device__ __forceinline__ float act_gelu_tanh(float g) {
@@ -372,7 +330,8 @@ hipError_t launch_norm(int op, const float *a, const float *b, const float *w, c
 // the caller (lt_api.cpp) before these are called.
 hipError_t launch_matvec_q4k(const DevTensor &W, const float *x, float *y, hipStream_t s);
 // Q8_0, and Q4_K / Q6_K rows of any length (lt_matvec.hip); the launchers
-// above and below take the K-quant rows they stream themselves.
+// above and below take the K-quant rows they stream, and small Q8_0 matrices,
+// themselves.
 hipError_t launch_matvec_rows(const DevTensor &W, const float *x, float *y, hipStream_t s);
 hipError_t launch_matvec_q8_0(const DevTensor &W, const float *x, float *y, hipStream_t s);
 hipError_t launch_matvec_q6k(const DevTensor &W, const float *x, float *y, hipStream_t s);

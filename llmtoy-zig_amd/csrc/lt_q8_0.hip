@@ -42,7 +42,8 @@ __device__ __forceinline__ void load_x16(const float *xs, int u, float *xv) {
 
 }  // namespace
 
-// y[r] = W[r] . x  (single) or h[r] = act(Wg[r] . x) * (Wu[r] . x)  (DUAL).
+// h[r] = act(Wg[r] . x) * (Wu[r] . x)  (DUAL), or y[r] = W[r] . x for small
+// matrices with rows of up to 3,072 elements.
 // G lanes per row, CPL units per lane, R rows per lane group; 256 threads.
 template <int G, int CPL, int R, bool DUAL>
 __global__ void __launch_bounds__(256) k_matvec_q8_0(const uint8_t *__restrict__ qa, const uint16_t *__restrict__ da,
@@ -102,22 +103,23 @@ static hipError_t launch_q8_t(const DevTensor &A, const DevTensor *B, const floa
                               hipStream_t s) {
     const int nrows = (int)A.total_rows, nb = (int)A.blocks_per_row;
     const int groups = 256 / G;
-    // fewer rows per group when the matrix is short, so the grid still covers the chip
-    const int R = (nrows >= groups * 4 * 512) ? 4 : (nrows >= groups * 2 * 512 ? 2 : 1);
+    // fewer rows per group when the matrix is short, so the grid still covers
+    // the chip (a single matrix here always is)
+    const int R = !DUAL ? 1 : (nrows >= groups * 4 * 512) ? 4 : (nrows >= groups * 2 * 512 ? 2 : 1);
     const int nblk = (nrows + groups * R - 1) / (groups * R);
     const uint8_t *qb = DUAL ? B->p0 : nullptr;
     const uint16_t *db = DUAL ? (const uint16_t *)B->p1 : nullptr;
     const size_t lds = (size_t)nb * 32 * sizeof(float);
-    if (R == 4)
-        hipLaunchKernelGGL((k_matvec_q8_0<G, CPL, 4, DUAL>), dim3(nblk), dim3(256), lds, s, A.p0,
-                           (const uint16_t *)A.p1, qb, db, x, y, nrows, nb, act);
-    else if (R == 2)
-        hipLaunchKernelGGL((k_matvec_q8_0<G, CPL, 2, DUAL>), dim3(nblk), dim3(256), lds, s, A.p0,
-                           (const uint16_t *)A.p1, qb, db, x, y, nrows, nb, act);
-    else
-        hipLaunchKernelGGL((k_matvec_q8_0<G, CPL, 1, DUAL>), dim3(nblk), dim3(256), lds, s, A.p0,
-                           (const uint16_t *)A.p1, qb, db, x, y, nrows, nb, act);
-    return hipGetLastError();
+    auto go = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(nblk), dim3(256), lds, s, A.p0, (const uint16_t *)A.p1, qb, db, x, y, nrows, nb,
+                           act);
+        return hipGetLastError();
+    };
+    if constexpr (DUAL) {
+        if (R == 4) return go(k_matvec_q8_0<G, CPL, 4, DUAL>);
+        if (R == 2) return go(k_matvec_q8_0<G, CPL, 2, DUAL>);
+    }
+    return go(k_matvec_q8_0<G, CPL, 1, DUAL>);
 }
 
 template <bool DUAL>
@@ -127,25 +129,28 @@ static hipError_t launch_q8_any(const DevTensor &A, const DevTensor *B, const fl
     if (nu <= 8) return launch_q8_t<8, 1, DUAL>(A, B, x, y, act, s);
     if (nu <= 16) return launch_q8_t<16, 1, DUAL>(A, B, x, y, act, s);
     if (nu <= 32) return launch_q8_t<32, 1, DUAL>(A, B, x, y, act, s);
-    switch ((nu + 63) / 64) {
-    case 1: return launch_q8_t<64, 1, DUAL>(A, B, x, y, act, s);
-    case 2: return launch_q8_t<64, 2, DUAL>(A, B, x, y, act, s);
-    case 3: return launch_q8_t<64, 3, DUAL>(A, B, x, y, act, s);
-    case 4: return launch_q8_t<64, 4, DUAL>(A, B, x, y, act, s);
-    case 5: return launch_q8_t<64, 5, DUAL>(A, B, x, y, act, s);
-    case 6: return launch_q8_t<64, 6, DUAL>(A, B, x, y, act, s);
-    case 7: return launch_q8_t<64, 7, DUAL>(A, B, x, y, act, s);
-    case 8: return launch_q8_t<64, 8, DUAL>(A, B, x, y, act, s);
-    case 9: return launch_q8_t<64, 9, DUAL>(A, B, x, y, act, s);
-    case 10: return launch_q8_t<64, 10, DUAL>(A, B, x, y, act, s);
-    case 11: return launch_q8_t<64, 11, DUAL>(A, B, x, y, act, s);
-    case 12: return launch_q8_t<64, 12, DUAL>(A, B, x, y, act, s);
-    case 13: return launch_q8_t<64, 13, DUAL>(A, B, x, y, act, s);
-    case 14: return launch_q8_t<64, 14, DUAL>(A, B, x, y, act, s);
-    case 15: return launch_q8_t<64, 15, DUAL>(A, B, x, y, act, s);
-    case 16: return launch_q8_t<64, 16, DUAL>(A, B, x, y, act, s);
-    default: return hipErrorInvalidValue;  // K > 16384: rejected by the API layer
+    if (nu <= 64) return launch_q8_t<64, 1, DUAL>(A, B, x, y, act, s);
+    if (nu <= 128) return launch_q8_t<64, 2, DUAL>(A, B, x, y, act, s);
+    if (nu <= 192) return launch_q8_t<64, 3, DUAL>(A, B, x, y, act, s);
+    if constexpr (DUAL) {
+        switch ((nu + 63) / 64) {
+        case 4: return launch_q8_t<64, 4, DUAL>(A, B, x, y, act, s);
+        case 5: return launch_q8_t<64, 5, DUAL>(A, B, x, y, act, s);
+        case 6: return launch_q8_t<64, 6, DUAL>(A, B, x, y, act, s);
+        case 7: return launch_q8_t<64, 7, DUAL>(A, B, x, y, act, s);
+        case 8: return launch_q8_t<64, 8, DUAL>(A, B, x, y, act, s);
+        case 9: return launch_q8_t<64, 9, DUAL>(A, B, x, y, act, s);
+        case 10: return launch_q8_t<64, 10, DUAL>(A, B, x, y, act, s);
+        case 11: return launch_q8_t<64, 11, DUAL>(A, B, x, y, act, s);
+        case 12: return launch_q8_t<64, 12, DUAL>(A, B, x, y, act, s);
+        case 13: return launch_q8_t<64, 13, DUAL>(A, B, x, y, act, s);
+        case 14: return launch_q8_t<64, 14, DUAL>(A, B, x, y, act, s);
+        case 15: return launch_q8_t<64, 15, DUAL>(A, B, x, y, act, s);
+        case 16: return launch_q8_t<64, 16, DUAL>(A, B, x, y, act, s);
+        default: break;
+        }
     }
+    return hipErrorInvalidValue;  // K > 16384: rejected by the API layer
 }
 
 hipError_t launch_matvec_q8_0(const DevTensor &W, const float *x, float *y, hipStream_t s) {
