@@ -423,8 +423,10 @@ hipError_t launch_expert_gate_up_q4k_routed(const DevTensor &GU, const float *x,
 // An output row is P = k U work units of 64 weights (slot s, unit u of the
 // slot's expert).  A thread keeps one of these positions, with its slot's 64
 // activations in registers (lt_rows.h), and a workgroup of RP = threads / P
-// rows side by side walks the output rows, the next pass's weights on their
-// way while the partial sums of this one meet in LDS: a slot's U units are
+// rows side by side walks the output rows; where it has several passes (more
+// rows than the workgroups of the chip hold at once: 2,048 x 768 at 8 slots is
+// one pass for each of 512), the next one's weights are on their way while the
+// partial sums of this one meet in LDS: a slot's U units are
 // added in order, then the slots in order, so the result does not depend on
 // scheduling.  Two rows per workgroup, with the activations read again by every
 // workgroup and a 16-byte header by every lane, took 7.8 us for 8 slots of
