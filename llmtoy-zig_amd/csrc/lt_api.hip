@@ -360,7 +360,8 @@ __global__ void __launch_bounds__(256) k_host_copy(const uint4 *__restrict__ src
 // context's pinned memory and a kernel: a pageable hipMemcpyAsync costs the
 // call more than the transfer (MoE layer of 2,048 on host buffers: 40.2 us
 // with pageable copies, 32.6 here).  Larger blocks, which the runtime
-// pipelines, go as before.
+// pipelines, go as pageable copies, and so do the norms' and the Gemma4 block's
+// vectors (io_in) and a selection on its way out (copy_routing_out).
 constexpr size_t kHostVec = 64 << 10, kPinBytes = 4 * kHostVec;
 
 int host_copy(lt_ctx *ctx, const void *src, void *dst, size_t bytes) {
