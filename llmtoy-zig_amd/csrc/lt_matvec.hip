@@ -123,12 +123,12 @@ hipError_t launch_rows_t(const DevTensor &W, const float *x, float *y, RowsPlan 
 
 // A launch of nt threads a workgroup and nd load buffers, on up to waves
 // wavefronts a CU.
-RowsPlan rows_plan(const DevTensor &W, int U, int nt, int nd, int waves) {
+RowsPlan rows_plan(int rows, int U, int nt, int nd, int waves) {
     RowsPlan p{};
     p.U = U;
     p.nthreads = nt;
     p.RP = nt / U;
-    p.npass = (int)((W.total_rows + p.RP - 1) / p.RP);
+    p.npass = (rows - 1) / p.RP + 1;
     p.nblk = std::min(p.npass, 256 * (waves * 64 / nt));
     p.nd = nd;
     return p;
@@ -142,31 +142,30 @@ RowsPlan rows_plan(const DevTensor &W, int U, int nt, int nd, int waves) {
 // a thread that go ahead of the weights.  Fitted to 570 sizes: the shape of
 // the least estimate takes 1.03 of the best shape's time on the average.
 template <class F>
-double rows_cost(const DevTensor &W, RowsPlan p) {
-    const int lds = (int)W.cols * 4 + p.nd * 4096;  // of a workgroup
-    p.nblk = std::min(p.nblk, 256 * ((160 << 10) / lds));
-    int passes = 0;
-    for (int b = 0; b < p.nblk; b += 256) {
-        const int n = (p.npass - b + p.nblk - 1) / p.nblk;
-        passes += (n + p.nd - 1) / p.nd * p.nd;
+double rows_cost(const RowsPlan &p, int cols, double row_bytes) {
+    // workgroups of that CU, as LDS (160 KB) lets them be resident
+    const int per_cu = std::min((p.nblk + 255) / 256, (160 << 10) / (cols * 4 + p.nd * 4096));
+    auto whole = [&](int n) { return (n + p.nd - 1) & ~(p.nd - 1); };  // passes in whole rounds
+    int passes = per_cu * p.nd;
+    double few = 1.0;
+    if (p.npass > 256 * per_cu) {
+        const int n = p.npass / (256 * per_cu), more = (p.npass - n * 256 * per_cu + 255) / 256;
+        passes = more * whole(n + 1) + (per_cu - more) * whole(n);
+        few = std::max(1.0, F::kLanes / (per_cu * p.RP * p.U));
     }
-    double t = (double)p.RP * passes * (W.bytes / W.total_rows) * (p.nd > 1 ? F::kRound : 1.0);
-    if (p.npass > p.nblk) {
-        const double few = std::max(1.0, F::kLanes / (p.nblk / 256 * p.RP * p.U));
-        t *= few * few * few;
-    }
-    const int late = std::max(0, ((int)W.cols / 4 - 2 * p.nthreads + p.nthreads - 1) / p.nthreads);
-    return t + 2.0 * ((p.nblk + 255) / 256) * W.cols * 4 + 3000.0 * late;
+    const int late = std::max(0, (cols / 4 - p.nthreads - 1) / p.nthreads);
+    return passes * (p.RP * row_bytes) * (p.nd > 1 ? F::kRound : 1.0) * (few * few * few) + 8.0 * per_cu * cols +
+           3000.0 * late;
 }
 
 template <class F>
 hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t s) {
-    const int U = (int)W.cols / F::kElems;
+    const int cols = (int)W.cols, rows = (int)W.total_rows, U = cols / F::kElems;
     // row indices are ints, and a last round's go up to 2 ND cap passes (2^21 rows) past the end
     if (U > 512 || W.total_rows > ((size_t)1 << 31) - (1 << 22)) return hipErrorInvalidValue;
     // up to two passes a workgroup: one load buffer, as the others would load
     // rows again that nobody needs (Q8_0 4,096 x 4,096: 6.3 us, 7.1 with four)
-    auto runs = [&](int nt) { return rows_plan(W, U, nt, 1, 16).npass > 2 * 256 * (1024 / nt); };
+    auto runs = [&](int npass, int nt) { return npass > 2 * 256 * (1024 / nt); };
     // The workgroup size that leaves the fewest lanes idle, the largest of
     // them: x is staged once per workgroup (Q4_K 4,096 x 11,008 on 512 threads
     // 11.6 us, on 256 14.9; Q8_0 7,001 x 2,816 7.6 and 8.2).  A short matrix
@@ -178,9 +177,10 @@ hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t
     double best = 0;
     RowsPlan p{};
     for (int nt = 512; nt >= 128 && nt >= U; nt -= 64) {
-        const RowsPlan q = rows_plan(W, U, nt, runs(nt) ? F::ND : 1, 16);
+        RowsPlan q = rows_plan(rows, U, nt, 1, 16);
+        if (runs(q.npass, nt)) q.nd = F::ND;
         const double used = (double)(q.RP * U) / nt * (q.npass >= 160 ? 1.0 : q.npass / 160.0) *
-                            (W.cols <= (size_t)8 * nt ? 1.0 : W.cols <= (size_t)16 * nt ? 0.75 : 0.4);
+                            (cols <= 8 * nt ? 1.0 : cols <= 16 * nt ? 0.75 : 0.4);
         if (used > best * 1.01) {
             best = used;
             p = q;
@@ -195,13 +195,14 @@ hipError_t launch_rows(const DevTensor &W, const float *x, float *y, hipStream_t
     // 11,000 x 2,048 8.5 | 6.8, 2,816 x 4,864 7.2 | 6.4; the other way Q4_K 16,000 x
     // 1,792 6.6 | 7.1, Q6_K 11,000 x 1,536 6.3 | 6.6.
     if (p.npass <= F::kLong * p.nblk) {
-        double least =
-            F::kKeep * rows_cost<F>(W, rows_plan(W, U, p.nthreads, p.nd, p.nd == 1 ? F::waves(U) : 16));
+        const double row_bytes = (double)W.bytes / rows;
+        double least = F::kKeep * rows_cost<F>(rows_plan(rows, U, p.nthreads, p.nd, p.nd == 1 ? F::waves(U) : 16), cols,
+                                               row_bytes);
         for (int nt = 512; nt >= 128 && nt >= U; nt -= 64)
             for (int nd : {1, F::ND}) {
-                if (!F::takes(U, nd, runs(nt))) continue;
-                const RowsPlan q = rows_plan(W, U, nt, nd, nd == 1 ? F::waves(U) : 16);
-                const double cost = rows_cost<F>(W, q);
+                const RowsPlan q = rows_plan(rows, U, nt, nd, nd == 1 ? F::waves(U) : 16);
+                if (!F::takes(U, nd, runs(q.npass, nt))) continue;
+                const double cost = rows_cost<F>(q, cols, row_bytes);
                 if (cost < least) {
                     least = cost;
                     p = q;
